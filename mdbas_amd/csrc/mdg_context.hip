@@ -527,7 +527,7 @@ extern "C" void mdg_destroy(mdg_ctx *ctx)
                     ctx->ca, ctx->cb, ctx->rc2, ctx->dd, ctx->grpAtomOff, ctx->grpAtoms,
                     ctx->grpConOff, ctx->grpCons, ctx->grpCycle, ctx->grpVir, ctx->ctrl,
                     ctx->exOff, ctx->exLst, ctx->xu, ctx->yu, ctx->zu, ctx->cellOf, ctx->cellCnt,
-                    ctx->cellStart, ctx->lcKeys, ctx->lcS3, ctx->rl.neighList, ctx->rl.neighPair,
+                    ctx->cellStart, ctx->lcKeys, ctx->lcS3, ctx->rl.neighList, ctx->refAtoms, ctx->rl.neighPair,
                     ctx->rl.neighOrder, ctx->rl.cnt, ctx->rl.off, ctx->cl.slotAtom,
                     ctx->cl.atomSlot, ctx->cl.bb, ctx->cl.bbh, ctx->cl.cpOff, ctx->cl.cpJ,
                     ctx->cl.cpMask, ctx->cl.cpI, ctx->cl.tmpCnt, ctx->cl.tmpJ, ctx->cl.tmpMask,
@@ -744,6 +744,7 @@ extern "C" int mdg_set_topology(mdg_ctx *ctx, const double q[], const double eps
     if (frozen) {
         RETCHK(h2d(ctx, ctx->frozen, frozen, n));
         for (int i = 0; i < n; i++) ctx->hasFrozen |= frozen[i] != 0;
+        ctx->listFrozen = ctx->hasFrozen;
     }
     if (nAtConst) RETCHK(h2d(ctx, ctx->nAtConst, nAtConst, n));
     charge_sums(ctx, q);
@@ -847,6 +848,7 @@ extern "C" int mdg_makelist(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, MDG_
         ctrl->keyLink = ctx->keyLink;
         if (frozen) {
             RETCHK(h2d(ctx, ctx->frozen, (const int *)frozen, n));
+            ctx->listFrozen = std::any_of(frozen, frozen + n, [](int f) { return f != 0; });
         }
         std::vector<int> l14;
         RETCHK(mdg_build_exclusions(ctx, param->nBond, bond, ctrl->keyConstH ? param->nConst : 0,

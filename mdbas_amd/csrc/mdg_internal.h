@@ -51,6 +51,12 @@ struct MdgParams {
                                  // (s_setprio); 2: the cluster pair kernel does
 };
 
+// One atom for the reference-list pair kernel: position and charge, then
+// eps, sig and padding to a 64-byte record.
+struct __align__(64) RefAtom {
+    double4 r, s;
+};
+
 // Reference-format list on the device.
 struct RefList {
     int *neighList = nullptr;    // flat j indices, in neighOrder order of i
@@ -214,6 +220,8 @@ struct mdg_ctx {
     double *q = nullptr, *eps = nullptr, *sig = nullptr, *mass = nullptr, *rmass = nullptr;
     int *frozen = nullptr, *nAtConst = nullptr;
     bool hasFrozen = false;
+    bool listFrozen = false;     // the device's frozen flags hold a non-zero one (mdg_makelist
+                                 // uploads them too)
     int nConst = 0;
     int *ca = nullptr, *cb = nullptr;
     double *rc2 = nullptr;
@@ -253,6 +261,7 @@ struct mdg_ctx {
     double *lcS3 = nullptr;
 
     RefList rl;
+    RefAtom *refAtoms = nullptr;   // drop-in pair loop: packed per atom records
     ClusterList cl;
     MdgBonded bd;
 
@@ -551,13 +560,18 @@ __device__ inline void mdg_block_max(double v, double *out)
 // ---------------------------------------------------------------- internal API
 void mdg_box_from(const MDG_PBC *in, MdgBox &b);
 void mdg_params_from(const MDG_CTRL *ctrl, const MDG_PARAM *p, MdgParams &P);
-// the reference-list pair kernel (k_pair_ref64) on a stream: per-block
-// partials [eElec, eVdw, virElec, virVdw, nIn, nListed] into part
+// the reference-list pair kernel (k_pair_ref64) on a stream, over packed atom
+// records: per-block partials [eElec, eVdw, virElec, virVdw, nIn, nListed]
+// into part, mdg_ref64_blocks(n) rows.  Up to 4 rows of the list a block;
+// from 16,384 on the wavefronts loop, which keeps the partials few.
+#define MDG_REF_MAX_BLOCKS 4096
+inline int mdg_ref64_blocks(int n) { return std::min(nblk(n, 4), MDG_REF_MAX_BLOCKS); }
+int mdg_ref_pack_launch(hipStream_t stream, int n, const double *x, const double *y,
+                        const double *z, const double *q, const double *eps, const double *sig,
+                        RefAtom *at);
 int mdg_pair_ref64_launch(hipStream_t stream, const MdgParams &P, const MdgBox &B, int elecType,
-                          const double *x, const double *y, const double *z, const double *q,
-                          const double *eps, const double *sig, const int *neighList,
-                          const long *off, const int *order, double *fx, double *fy, double *fz,
-                          double *part);
+                          const RefAtom *at, const int *neighList, const long *off,
+                          const int *order, double *fx, double *fy, double *fz, double *part);
 int mdg_reduce_partials_on(hipStream_t stream, const double *part, int nblocks, int nv,
                            double *out);
 int mdg_alloc_state(mdg_ctx *ctx);

@@ -130,33 +130,40 @@ __global__ void k_segment_sort(unsigned long long *__restrict__ keys, const int 
 
 // ---------------------------------------------------------------- O(N^2)
 
-// list.c:896-1040 count / fill passes, one thread per i (rows ascending).
+// list.c:896-1040 count / fill passes, one wavefront per i (rows ascending):
+// the lanes test 64 consecutive j and a ballot gives each hit its place, so
+// the row keeps the reference's order.  The exclusion table is searched only
+// within the widest excluded span.  One thread per i took 1,190 and 1,369 us
+// (count, fill) at 3,000 atoms: 12 blocks, a row's j one after the other.
 template <bool FILL>
-__global__ void k_verlet(MdgParams P, MdgBox B, const double *__restrict__ x,
-                         const double *__restrict__ y, const double *__restrict__ z,
-                         const int *__restrict__ frozen, const int *__restrict__ exOff,
-                         const int *__restrict__ exLst, int *__restrict__ cnt,
-                         const long *__restrict__ off, int *__restrict__ neighList)
+__global__ void __launch_bounds__(256)
+k_verlet(MdgParams P, MdgBox B, const double *__restrict__ x, const double *__restrict__ y,
+         const double *__restrict__ z, bool hasFrozen, const int *__restrict__ frozen,
+         const int *__restrict__ exOff, const int *__restrict__ exLst, int exSpan,
+         int *__restrict__ cnt, const long *__restrict__ off, int *__restrict__ neighList)
 {
 #pragma clang fp contract(off)
-    int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int i = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
     if (i >= P.n) return;
     const double xi = x[i], yi = y[i], zi = z[i];
-    const int fi = frozen[i];
+    const int fi = hasFrozen ? frozen[i] : 0;
     int c = 0;
-    long o = FILL ? off[i] : 0;
-    for (int j = i + 1; j < P.n; j++) {
-        double dx = x[j] - xi, dy = y[j] - yi, dz = z[j] - zi;
-        double r2 = mdg_dist(B, dx, dy, dz);
-        if (r2 <= P.cutnb2) {
-            bool ex = (fi * frozen[j]) ? true : mdg_excluded(exOff, exLst, i, j);
-            if (!ex) {
-                if (FILL) neighList[o + c] = j;
-                c++;
-            }
+    const long o = FILL ? off[i] : 0;
+    for (int j0 = i + 1; j0 < P.n; j0 += 64) {
+        const int j = j0 + lane;
+        bool hit = false;
+        if (j < P.n) {
+            double dx = x[j] - xi, dy = y[j] - yi, dz = z[j] - zi;
+            hit = mdg_dist(B, dx, dy, dz) <= P.cutnb2;
+            if (hit && hasFrozen && fi * frozen[j]) hit = false;
+            if (hit && j - i <= exSpan) hit = !mdg_excluded(exOff, exLst, i, j);
         }
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
+        if (FILL && hit) neighList[o + c + __builtin_popcountll(m & ((1ull << lane) - 1))] = j;
+        c += __builtin_popcountll(m);
     }
-    if (!FILL) cnt[i] = c;
+    if (!FILL && lane == 0) cnt[i] = c;
 }
 
 __global__ void k_identity(int n, int *order, const int *cnt, int *neighPair)
@@ -229,58 +236,125 @@ __constant__ int c_tx[14] = {0, 1, 0, 0, -1, 1, 0, -1, 1, 0, -1, 1, -1, 1};
 __constant__ int c_ty[14] = {0, 0, 1, 0, 1, 1, -1, 0, 0, 1, -1, -1, 1, 1};
 __constant__ int c_tz[14] = {0, 0, 0, 1, 0, 0, 1, 1, 1, 1, 1, 1, 1, 1};
 
+// Bounding box, in scaled coordinates, of each aligned run of 64 positions
+// of the cell order (lo x, y, z, hi x, y, z): one wavefront per run.
+__global__ void __launch_bounds__(256)
+k_lc_runs(int n, const double *__restrict__ sxu, const double *__restrict__ syu,
+          const double *__restrict__ szu, double *__restrict__ run)
+{
+    const int lane = threadIdx.x & 63;
+    const int r = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (r * 64 >= n) return;
+    const int p = min(r * 64 + lane, n - 1);
+    const double v[3] = {sxu[p], syu[p], szu[p]};
+#pragma unroll
+    for (int d = 0; d < 3; d++) {
+        double lo = v[d], hi = v[d];
+        for (int o = 32; o > 0; o >>= 1) {
+            lo = fmin(lo, __shfl_xor(lo, o, 64));
+            hi = fmax(hi, __shfl_xor(hi, o, 64));
+        }
+        if (lane == 0) {
+            run[(long)r * 6 + d] = lo;
+            run[(long)r * 6 + 3 + d] = hi;
+        }
+    }
+}
+
 // list.c:2130-2261: for position p (atom i in cell k), the 14 half-shell
 // cells in table order; j runs over the cell's chain, or over the chain
-// after i in i's own cell.  Count pass and fill pass.
+// after i in i's own cell.  Count pass and fill pass, one wavefront per
+// position: for each cell the lanes first test the bounding boxes of its
+// runs of 64 positions (at most 64 runs at a time), then walk the runs that
+// can hold a pair, 64 j at a time; a ballot gives each hit its place, so the
+// row keeps the reference's order.  Bound by the FP64 distance tests: a cell
+// is 14 to 20 A wide, about one candidate in nine is a pair.  A run is left
+// out only when its box lies beyond the cutoff by more than the rounding of
+// the test (rectangular boxes).  One thread per position, its j one after
+// the other, took 2,428 and 2,770 us (count, fill) at 30,000 atoms.
 template <bool FILL>
-__global__ void k_lc_pairs(MdgParams P, MdgBox B, int nx, int ny, int nz,
-                           const int *__restrict__ order, const int *__restrict__ cellOf,
-                           const int *__restrict__ cellStart, const double *__restrict__ sxu,
-                           const double *__restrict__ syu, const double *__restrict__ szu,
-                           const int *__restrict__ frozen, const int *__restrict__ exOff,
-                           const int *__restrict__ exLst, int *__restrict__ cnt,
-                           const long *__restrict__ off, int *__restrict__ neighList,
-                           int *__restrict__ neighPair)
+__global__ void __launch_bounds__(256)
+k_lc_pairs(MdgParams P, MdgBox B, int nx, int ny, int nz, const int *__restrict__ order,
+           const int *__restrict__ cellOf, const int *__restrict__ cellStart,
+           const double *__restrict__ sxu, const double *__restrict__ syu,
+           const double *__restrict__ szu, const double *__restrict__ run, bool hasFrozen,
+           const int *__restrict__ frozen, const int *__restrict__ exOff,
+           const int *__restrict__ exLst, int exSpan, int *__restrict__ cnt,
+           const long *__restrict__ off, int *__restrict__ neighList, int *__restrict__ neighPair)
 {
 #pragma clang fp contract(off)
-    int p = blockIdx.x * blockDim.x + threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int p = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
     if (p >= P.n) return;
     const int i = order[p];
     const int k = cellOf[i];
     const int ix = k % nx, iy = (k / nx) % ny, iz = k / (nx * ny);
     const double xi = sxu[p], yi = syu[p], zi = szu[p];
-    const int fi = frozen[i];
+    const int fi = hasFrozen ? frozen[i] : 0;
+    const bool rect = B.type != 3;
+    const double far2 = P.cutnb2 * (1. + 1e-9) + 1e-9;
     int c = 0;
-    long o = FILL ? off[p] : 0;
+    const long o = FILL ? off[p] : 0;
     for (int l = 0; l < 14; l++) {
         double cx = 0., cy = 0., cz = 0.;
         int jx = ix + c_tx[l], jy = iy + c_ty[l], jz = iz + c_tz[l];
         if (jx > nx - 1) { jx -= nx; cx = 1.; } else if (jx < 0) { jx += nx; cx = -1.; }
         if (jy > ny - 1) { jy -= ny; cy = 1.; } else if (jy < 0) { jy += ny; cy = -1.; }
         if (jz > nz - 1) { jz -= nz; cz = 1.; } else if (jz < 0) { jz += nz; cz = -1.; }
-        int ll = jx + nx * (jy + ny * jz);
-        int q0 = (ll == k) ? p + 1 : cellStart[ll];
-        int q1 = cellStart[ll + 1];
-        for (int q = q0; q < q1; q++) {
-            double xt = sxu[q] - xi + cx;
-            double yt = syu[q] - yi + cy;
-            double zt = szu[q] - zi + cz;
-            double xd = xt * B.a1 + yt * B.b1 + zt * B.c1;
-            double yd = xt * B.a2 + yt * B.b2 + zt * B.c2;
-            double zd = xt * B.a3 + yt * B.b3 + zt * B.c3;
-            double r2 = xd * xd + yd * yd + zd * zd;
-            if (r2 <= P.cutnb2) {
-                int j = order[q];
-                bool ex = (fi * frozen[j]) ? true : mdg_excluded(exOff, exLst, i, j);
-                if (!ex) {
-                    if (FILL) neighList[o + c] = j;
-                    c++;
+        const int ll = jx + nx * (jy + ny * jz);
+        const int q0 = (ll == k) ? p + 1 : cellStart[ll];
+        const int q1 = cellStart[ll + 1];
+        for (int r0 = q0 >> 6; r0 * 64 < q1; r0 += 64) {
+            const int r = r0 + lane;
+            bool near = q0 < q1 && r * 64 < q1;
+            if (near && rect) {
+                const double *b = run + (long)r * 6;
+                const double dx = fmax(fmax(b[0] + cx - xi, xi - cx - b[3]), 0.) * B.a1;
+                const double dy = fmax(fmax(b[1] + cy - yi, yi - cy - b[4]), 0.) * B.b2;
+                const double dz = fmax(fmax(b[2] + cz - zi, zi - cz - b[5]), 0.) * B.c3;
+                near = dx * dx + dy * dy + dz * dz <= far2;
+            }
+            unsigned long long runs = __builtin_amdgcn_ballot_w64(near);
+            while (runs) {
+                const int q = (r0 + __builtin_ctzll(runs)) * 64 + lane;
+                runs &= runs - 1;
+                bool hit = false;
+                if (q >= q0 && q < q1) {
+                    const double xt = sxu[q] - xi + cx;
+                    const double yt = syu[q] - yi + cy;
+                    const double zt = szu[q] - zi + cz;
+                    double xd, yd, zd;
+                    if (rect) {
+                        // the off-diagonal terms are products with +-0: they
+                        // change at most the sign of a zero, which r2 drops
+                        xd = xt * B.a1;
+                        yd = yt * B.b2;
+                        zd = zt * B.c3;
+                    } else {
+                        xd = xt * B.a1 + yt * B.b1 + zt * B.c1;
+                        yd = xt * B.a2 + yt * B.b2 + zt * B.c2;
+                        zd = xt * B.a3 + yt * B.b3 + zt * B.c3;
+                    }
+                    hit = xd * xd + yd * yd + zd * zd <= P.cutnb2;
                 }
+                int j = 0;
+                if (hit) {
+                    j = order[q];
+                    if (hasFrozen && fi * frozen[j]) hit = false;
+                    const int s = j - i;
+                    if (hit && (s < 0 ? -s : s) <= exSpan) hit = !mdg_excluded(exOff, exLst, i, j);
+                }
+                const unsigned long long m = __builtin_amdgcn_ballot_w64(hit);
+                if (FILL && hit)
+                    neighList[o + c + __builtin_popcountll(m & ((1ull << lane) - 1))] = j;
+                c += __builtin_popcountll(m);
             }
         }
     }
-    if (!FILL) cnt[p] = c;
-    else neighPair[i] = c;
+    if (lane == 0) {
+        if (!FILL) cnt[p] = c;
+        else neighPair[i] = c;
+    }
 }
 
 static int ensure_int(mdg_ctx *ctx, int **p, size_t n)
@@ -343,16 +417,23 @@ int mdg_build_ref_list(mdg_ctx *ctx, bool wrap)
             LAUNCHCHK();
         }
         if (!ctx->lcKeys) HIPCHK(hipMalloc(&ctx->lcKeys, n * sizeof(unsigned long long)));
-        if (!ctx->lcS3) HIPCHK(hipMalloc(&ctx->lcS3, 3 * (size_t)n * sizeof(double)));
+        // scaled coordinates in cell order, then the boxes of its 64-position runs
+        const int nrun = nblk(n, 64);
+        if (!ctx->lcS3)
+            HIPCHK(hipMalloc(&ctx->lcS3, (3 * (size_t)n + 6 * (size_t)nrun) * sizeof(double)));
         unsigned long long *keys = ctx->lcKeys;
         double *s3 = ctx->lcS3;
         double *sxu = s3, *syu = s3 + n, *szu = s3 + 2 * n;
         RETCHK(lc_sort(ctx, &keys, &sxu, &syu, &szu));
         const int nx = ctx->nlc[0], ny = ctx->nlc[1], nz = ctx->nlc[2];
-        hipLaunchKernelGGL((k_lc_pairs<false>), dim3(nblk(n, 128)), dim3(128), 0, ctx->stream,
+        double *run = s3 + 3 * (size_t)n;
+        hipLaunchKernelGGL(k_lc_runs, dim3(nblk(nrun, 4)), dim3(256), 0, ctx->stream, n, sxu, syu,
+                           szu, run);
+        LAUNCHCHK();
+        hipLaunchKernelGGL((k_lc_pairs<false>), dim3(nblk(n, 4)), dim3(256), 0, ctx->stream,
                            ctx->P, ctx->B, nx, ny, nz, R.neighOrder, ctx->cellOf, ctx->cellStart,
-                           sxu, syu, szu, ctx->frozen, ctx->exOff, ctx->exLst, R.cnt, nullptr,
-                           nullptr, nullptr);
+                           sxu, syu, szu, run, ctx->listFrozen, ctx->frozen, ctx->exOff,
+                           ctx->exLst, ctx->exSpan, R.cnt, nullptr, nullptr, nullptr);
         LAUNCHCHK();
         RETCHK(mdg_scan_int_to_long(ctx, R.cnt, R.off, n));
         long total = 0;
@@ -364,15 +445,15 @@ int mdg_build_ref_list(mdg_ctx *ctx, bool wrap)
             HIPCHK(hipMalloc(&R.neighList, R.cap * sizeof(int)));
         }
         R.count = total;
-        hipLaunchKernelGGL((k_lc_pairs<true>), dim3(nblk(n, 128)), dim3(128), 0, ctx->stream,
+        hipLaunchKernelGGL((k_lc_pairs<true>), dim3(nblk(n, 4)), dim3(256), 0, ctx->stream,
                            ctx->P, ctx->B, nx, ny, nz, R.neighOrder, ctx->cellOf, ctx->cellStart,
-                           sxu, syu, szu, ctx->frozen, ctx->exOff, ctx->exLst, R.cnt, R.off,
-                           R.neighList, R.neighPair);
+                           sxu, syu, szu, run, ctx->listFrozen, ctx->frozen, ctx->exOff,
+                           ctx->exLst, ctx->exSpan, R.cnt, R.off, R.neighList, R.neighPair);
         LAUNCHCHK();
     } else {
-        hipLaunchKernelGGL((k_verlet<false>), dim3(nblk(n, 128)), dim3(128), 0, ctx->stream,
-                           ctx->P, ctx->B, ctx->x, ctx->y, ctx->z, ctx->frozen, ctx->exOff,
-                           ctx->exLst, R.cnt, nullptr, nullptr);
+        hipLaunchKernelGGL((k_verlet<false>), dim3(nblk(n, 4)), dim3(256), 0, ctx->stream,
+                           ctx->P, ctx->B, ctx->x, ctx->y, ctx->z, ctx->listFrozen, ctx->frozen,
+                           ctx->exOff, ctx->exLst, ctx->exSpan, R.cnt, nullptr, nullptr);
         LAUNCHCHK();
         RETCHK(mdg_scan_int_to_long(ctx, R.cnt, R.off, n));
         long total = 0;
@@ -384,9 +465,9 @@ int mdg_build_ref_list(mdg_ctx *ctx, bool wrap)
             HIPCHK(hipMalloc(&R.neighList, R.cap * sizeof(int)));
         }
         R.count = total;
-        hipLaunchKernelGGL((k_verlet<true>), dim3(nblk(n, 128)), dim3(128), 0, ctx->stream,
-                           ctx->P, ctx->B, ctx->x, ctx->y, ctx->z, ctx->frozen, ctx->exOff,
-                           ctx->exLst, nullptr, R.off, R.neighList);
+        hipLaunchKernelGGL((k_verlet<true>), dim3(nblk(n, 4)), dim3(256), 0, ctx->stream,
+                           ctx->P, ctx->B, ctx->x, ctx->y, ctx->z, ctx->listFrozen, ctx->frozen,
+                           ctx->exOff, ctx->exLst, ctx->exSpan, nullptr, R.off, R.neighList);
         LAUNCHCHK();
         hipLaunchKernelGGL(k_identity, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, n,
                            R.neighOrder, R.cnt, R.neighPair);
