@@ -562,10 +562,16 @@ void mdg_box_from(const MDG_PBC *in, MdgBox &b);
 void mdg_params_from(const MDG_CTRL *ctrl, const MDG_PARAM *p, MdgParams &P);
 // the reference-list pair kernel (k_pair_ref64) on a stream, over packed atom
 // records: per-block partials [eElec, eVdw, virElec, virVdw, nIn, nListed]
-// into part, mdg_ref64_blocks(n) rows.  Up to 4 rows of the list a block;
-// from 16,384 on the wavefronts loop, which keeps the partials few.
-#define MDG_REF_MAX_BLOCKS 4096
-inline int mdg_ref64_blocks(int n) { return std::min(nblk(n, 4), MDG_REF_MAX_BLOCKS); }
+// into part, mdg_ref64_blocks(n) rows.  A block takes mdg_ref64_group(n) rows
+// of the list: whole rounds of the 256 CUs (a block fills one) with at most 32
+// rows a block, beyond which a group's distinct j outgrow its LDS table, and at
+// least 4, below which rows would share too few j to collect.
+inline int mdg_ref64_group(int n)
+{
+    const int rounds = nblk(n, 256 * 32);
+    return std::max(nblk(n, 256 * rounds), 4);
+}
+inline int mdg_ref64_blocks(int n) { return nblk(n, mdg_ref64_group(n)); }
 int mdg_ref_pack_launch(hipStream_t stream, int n, const double *x, const double *y,
                         const double *z, const double *q, const double *eps, const double *sig,
                         RefAtom *at);

@@ -20,15 +20,16 @@
 namespace {
 constexpr int MAX_ATOMS = MDG_NOALLOC_MAX_ATOMS;
 constexpr int NV = 6;   // k_pair_ref64 partials per block
+constexpr int MAX_BLOCKS = MAX_ATOMS / 32 + 256;   // mdg_ref64_blocks at every size
 constexpr int SEG = 1024;   // list rows a block of the offset kernels scans
 constexpr int MAX_SEG = (MAX_ATOMS + SEG - 1) / SEG;
 // layout: list offsets (MAX_ATOMS + 1 longs), their segment sums (MAX_SEG
-// longs), partials (MDG_REF_MAX_BLOCKS x NV doubles), packed atom records
+// longs), partials (MAX_BLOCKS x NV doubles), packed atom records
 // (MAX_ATOMS x 64 bytes): 19 MB
 constexpr size_t up256(size_t b) { return (b + 255) / 256 * 256; }
 constexpr size_t OFF_BYTES = up256((size_t)(MAX_ATOMS + 1) * sizeof(long));
 constexpr size_t SEG_BYTES = up256((size_t)MAX_SEG * sizeof(long));
-constexpr size_t PART_BYTES = up256((size_t)MDG_REF_MAX_BLOCKS * NV * sizeof(double));
+constexpr size_t PART_BYTES = up256((size_t)MAX_BLOCKS * NV * sizeof(double));
 constexpr size_t SCRATCH_BYTES = OFF_BYTES + SEG_BYTES + PART_BYTES +
                                  (size_t)MAX_ATOMS * sizeof(RefAtom);
 }  // namespace

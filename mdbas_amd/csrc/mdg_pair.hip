@@ -117,24 +117,50 @@ __device__ __forceinline__ double ref_dist(const MdgBox &b, double &dx, double &
 
 // energies out per block: [eElec, eVdw, virElec, virVdw, nIn, nListed]
 //
-// One wavefront per row (the list's consecutive j of one i): the row is read
-// 64 entries at a time, coalesced, the j records are gathered one iteration
-// ahead, the i force stays in registers and is summed once per row.  Bound by
-// the FP64 issue of the pair arithmetic and the three force atomics of a pair.
-// One thread per row, as before, left all but 12 of 256 CUs idle at 3,000
-// atoms and read the list with a stride of a row between lanes: 1,645 us a
+// A block takes a group of consecutive rows (the list's consecutive j of one
+// i), a wavefront a row at a time: the row is read 64 entries at a time,
+// coalesced, the j records are gathered one iteration ahead, the i force stays
+// in registers and is summed once per row.
+//
+// j forces collect in LDS.  A pair's three FP64 force atomics to memory are
+// what bounds the plain form: 32 million of them at 30,000 atoms took 535 us
+// of 590 (about 60 a nanosecond, the same whether or not each XCD has its own
+// copy of the forces), the arithmetic and the list 136.  The rows of a group
+// are neighbours in space (the list's order is by cell), so they share most of
+// their j: a table of REF_SLOTS entries, two hashed places per j and the first
+// to claim a place keeps it, adds them up and goes to memory once per group.  A
+// j that finds both places taken adds to memory directly, so the table only
+// saves traffic and is never a limit.
+//
+// One thread per row, the form before that, left all but 12 of 256 CUs idle at
+// 3,000 atoms and read the list with a row's stride between lanes: 1,645 us a
 // call there and 1,746 us at 30,000 atoms (17.3 million entries).
+#define REF_SLOTS 4096
+#define REF_THREADS 1024
+
 template <int ELEC>
-__global__ void __launch_bounds__(256)
-k_pair_ref64(MdgParams P, MdgBox B, const RefAtom *__restrict__ at,
+__global__ void __launch_bounds__(REF_THREADS)
+k_pair_ref64(MdgParams P, MdgBox B, int group, const RefAtom *__restrict__ at,
              const int *__restrict__ neighList, const long *__restrict__ off,
              const int *__restrict__ order, double *fx, double *fy, double *fz,
              double *__restrict__ part)
 {
+    __shared__ double tx[REF_SLOTS], ty[REF_SLOTS], tz[REF_SLOTS];
+    __shared__ int tag[REF_SLOTS], nextRow;
+    for (int t = threadIdx.x; t < REF_SLOTS; t += REF_THREADS) {
+        tx[t] = ty[t] = tz[t] = 0.;
+        tag[t] = -1;
+    }
+    const int row0 = blockIdx.x * group, row1 = min(row0 + group, P.n);
+    if (threadIdx.x == 0) nextRow = row0;
+    __syncthreads();
     const int lane = threadIdx.x & 63;
     double acc[6] = {0, 0, 0, 0, 0, 0};
-    for (int l = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); l < P.n;
-         l += gridDim.x * 4) {
+    for (;;) {
+        int l = 0;
+        if (lane == 0) l = atomicAdd(&nextRow, 1);
+        l = __builtin_amdgcn_readfirstlane(l);
+        if (l >= row1) break;
         const long k0 = off[l], k1 = off[l + 1];
         if (k0 >= k1) continue;
         const int i = order[l];
@@ -157,6 +183,19 @@ k_pair_ref64(MdgParams P, MdgBox B, const RefAtom *__restrict__ at,
             nin += __builtin_popcountll(__builtin_amdgcn_ballot_w64(in));
             if (in) {
                 const double2 sj = *(const double2 *)&at[j].s;
+                // j's place in the table (-1: none)
+                const unsigned int h = (unsigned int)j * 2654435761u;
+                int slot = h >> 20;
+                int t = tag[slot];
+                if (t != j) {
+                    if (t < 0) t = atomicCAS(&tag[slot], -1, j);
+                    if (t >= 0 && t != j) {
+                        slot = (h >> 8) & (REF_SLOTS - 1);
+                        t = tag[slot];
+                        if (t < 0) t = atomicCAS(&tag[slot], -1, j);
+                        if (t >= 0 && t != j) slot = -1;
+                    }
+                }
                 double r;
                 const double rt = mdg_rsqrt64(r2, r);
                 double dEl, dVw = 0., el, ev = 0.;
@@ -172,9 +211,15 @@ k_pair_ref64(MdgParams P, MdgBox B, const RefAtom *__restrict__ at,
                 fxi += fxj;
                 fyi += fyj;
                 fzi += fzj;
-                atomicAdd(&fx[j], -fxj);
-                atomicAdd(&fy[j], -fyj);
-                atomicAdd(&fz[j], -fzj);
+                if (slot >= 0) {
+                    atomicAdd(&tx[slot], -fxj);
+                    atomicAdd(&ty[slot], -fyj);
+                    atomicAdd(&tz[slot], -fzj);
+                } else {
+                    atomicAdd(&fx[j], -fxj);
+                    atomicAdd(&fy[j], -fyj);
+                    atomicAdd(&fz[j], -fzj);
+                }
             }
             j = jn;
             jn = j2;
@@ -189,6 +234,14 @@ k_pair_ref64(MdgParams P, MdgBox B, const RefAtom *__restrict__ at,
             acc[4] += (double)nin;
             acc[5] += (double)(k1 - k0);
         }
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < REF_SLOTS; t += REF_THREADS) {
+        const int j = tag[t];
+        if (j < 0) continue;
+        atomicAdd(&fx[j], tx[t]);
+        atomicAdd(&fy[j], ty[t]);
+        atomicAdd(&fz[j], tz[t]);
     }
     mdg_block_partials<6>(acc, part);
 }
@@ -242,10 +295,10 @@ int mdg_pair_ref64_launch(hipStream_t stream, const MdgParams &P, const MdgBox &
                           const RefAtom *at, const int *neighList, const long *off,
                           const int *order, double *fx, double *fy, double *fz, double *part)
 {
-    const int nb = mdg_ref64_blocks(P.n);
+    const int nb = mdg_ref64_blocks(P.n), group = mdg_ref64_group(P.n);
 #define MDG_REF_LAUNCH(E)                                                                          \
-    hipLaunchKernelGGL(k_pair_ref64<E>, dim3(nb), dim3(256), 0, stream, P, B, at, neighList, off,  \
-                       order, fx, fy, fz, part)
+    hipLaunchKernelGGL(k_pair_ref64<E>, dim3(nb), dim3(REF_THREADS), 0, stream, P, B, group, at,   \
+                       neighList, off, order, fx, fy, fz, part)
     switch (elecType) {
     case 0: MDG_REF_LAUNCH(0); break;
     case 1: MDG_REF_LAUNCH(1); break;
