@@ -148,45 +148,21 @@ __device__ inline void shake_publish_mask_b(const ShakeArgs &A,
 }
 
 // First sweep index at which every group was converged (-1 if none); mask
-// is the run's (or one replica's) SHK_MASKW words.
+// is the run's (or one replica's) SHK_MASKW words, all requested at once.
 __device__ inline int shake_global_stop(const ShakeArgs &A, const unsigned long long *mask)
 {
-    for (int w = 0; w < SHK_MASKW; w++) {
-        unsigned long long m = mask[w];
-        if (m) {
-            int k = w * 64 + __ffsll((long long)m) - 1;
-            return k < A.P.maxCycle ? k : -1;
-        }
-    }
-    return -1;
+    unsigned long long m[SHK_MASKW];
+#pragma unroll
+    for (int w = 0; w < SHK_MASKW; w++) m[w] = mask[w];
+    int k = 64 * SHK_MASKW;
+#pragma unroll
+    for (int w = SHK_MASKW - 1; w >= 0; w--)
+        if (m[w]) k = w * 64 + __ffsll((long long)m[w]) - 1;
+    return k < A.P.maxCycle ? k : -1;
 }
 
 __device__ inline int shake_global_stop(const ShakeArgs &A) { return shake_global_stop(A, A.mask); }
 
-
-// Which saved state leads to sweep C: a window or ring slot, the end
-// state, or the start (when C lies outside both and before the end).  ring:
-// the group's SHK_R ring sweeps (-1 when empty).
-__device__ inline void shake_pick_slot(int C, int first, int kend, const int *ring, int &slot, int &at)
-{
-    int rs = -1;
-    if (ring)
-        for (int q = 0; q < SHK_R; q++)
-            if (ring[q] == C) rs = q;
-    if (first >= 0 && C >= first && C - first < SHK_W && C <= kend) {
-        slot = 1 + C - first;
-        at = C;
-    } else if (rs >= 0) {
-        slot = SHK_W + 2 + rs;
-        at = C;
-    } else if (C >= kend) {
-        slot = SHK_W + 1;
-        at = kend;
-    } else {
-        slot = 0;
-        at = 0;
-    }
-}
 
 // utils.c:162-218 (image_update) for one atom.
 __device__ inline void shake_image(const MdgBox &B, double &xs, double &ys, double &zs)
