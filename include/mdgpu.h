@@ -390,7 +390,9 @@ int mdg_autotune(mdg_ctx *ctx, int nsteps, int out[2]);
  * [1] pair grid cap, [2] 1 when steps without a rebuild enqueue the SPME
  * branch before the pair branch, [3] 1 when the binned SPME kernels raise
  * their wave priority above the pair kernel's beside them, 2 when the
- * mixed pair kernel raises its own instead.  mdg_set_launch
+ * mixed pair kernel raises its own instead.  The first list build picks
+ * [1] and [2] by the system's size unless mdg_set_launch came before it.
+ * mdg_set_launch
  * restores a saved set (per-atom results do not depend on them).  No
  * reference counterpart. */
 int mdg_get_launch(const mdg_ctx *ctx, int out[4]);
@@ -409,10 +411,10 @@ int mdg_phase_times(mdg_ctx *ctx, double out[5]);
  * kernel runs on that shorter list while no atom has moved more than
  * skin / 2 since, and on the full list otherwise.  Forces, energies and
  * virials are the same bit for bit either way.  skin = 0 switches it off;
- * it is capped at the list skin (delr).  Default for mixed contexts:
- * 0.8 A where every box edge exceeds 2 (cutOff + 0.8 A + 3 A), else off
- * (the prune kernel's test needs that room, and small boxes gain
- * little).  No reference counterpart: the reference evaluates every
+ * it is capped at the list skin (delr).  Default: off; mdg_autotune tries
+ * 0.8 A in mixed contexts where every box edge exceeds 2 (cutOff + 0.8 A +
+ * 3 A) (the prune kernel's test needs that room), unless this call has
+ * switched it off.  No reference counterpart: the reference evaluates every
  * listed pair (energy.c:480-541), which this reproduces. */
 int mdg_set_prune(mdg_ctx *ctx, double skin);
 double mdg_prune_skin(const mdg_ctx *ctx);   /* the current pruning distance */

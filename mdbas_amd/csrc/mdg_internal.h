@@ -16,8 +16,8 @@
 #define MDG_GRP_ATOMS 8          // max atoms in one constraint group
 #define MDG_GRP_CONS 16          // max constraints in one constraint group
 #define MDG_SEG_MAX 4096         // max atoms in one cell segment sorted in LDS
-#define MDG_CHUNK 32             // j-clusters per wavefront in the pair kernel
-#define MDG_PRUNE_SKIN 0.8       // default pruning distance beyond the cutoff (mixed), A
+#define MDG_CHUNK 32             // j-clusters per wavefront in the mixed pair kernel
+#define MDG_PRUNE_SKIN 0.8       // pruning distance beyond the cutoff the tuner tries (mixed), A
 
 // Fixed-point scales: forces in internal units (10 J/mol/A) carry 2^32
 // fractional steps in an int64 (|F| < 2^31); energies and virials 2^24
@@ -86,6 +86,7 @@ struct ClusterList {
     int *chOff = nullptr;        // per I: first chunk (nclu+1)
     int2 *chunk = nullptr;       // chunk -> (I, first entry)
     int maxChunks = 0;
+    int chunkLen = MDG_CHUNK;    // entries per chunk, set by the first build (chunk_len)
     int *tmpCnt = nullptr;       // per I: entries found
     int *tmpJ = nullptr;         // per I scratch [nclu][kmax]
     unsigned long long *tmpMask = nullptr;
@@ -182,6 +183,7 @@ struct MdgTune {
                                  // rebuild steps always do)
     int spmePrio = 0;            // 1: the binned SPME kernels' waves issue ahead of the pair
                                  // kernel's when both share a SIMD; 2: the pair kernel's ahead
+    bool set = false;            // chosen by mdg_set_launch or mdg_autotune: no default by size
 };
 
 struct mdg_ctx {
@@ -277,6 +279,7 @@ struct mdg_ctx {
     double *relPart = nullptr;
     int pairPath = 0;
     double pruneSkin = 0.;       // > 0: the mixed pair kernel may use the pruned list
+    bool pruneSet = false;       // mdg_set_prune was called: the tuner adds no pruning of its own
     bool pruneFresh = true;      // the list was rebuilt since the last slot update
     // device steps without a rebuild (one box of three-site molecules,
     // mixed): stage 1's replay kernel writes the slot positions
@@ -617,6 +620,7 @@ int mdg_excl_corr64(mdg_ctx *ctx, double *fx, double *fy, double *fz, double *eo
 int mdg_pair_cluster(mdg_ctx *ctx);
 int mdg_slot_params(mdg_ctx *ctx);
 int mdg_prune_list(mdg_ctx *ctx);   // mdg_pair.hip: refresh the pruned list (mixed)
+double mdg_prune_candidate(const mdg_ctx *ctx);   // mdg_context.hip: the skin the tuner tries
 
 // spme (mdg_spme.hip)
 int mdg_spme_setup(mdg_ctx *ctx);

@@ -896,19 +896,20 @@ __global__ void k_cluster_compact(int nclu, int kmax, const int *__restrict__ tm
     }
 }
 
-__global__ void k_chunk_count(int nclu, const int *__restrict__ tmpCnt, int *__restrict__ nch)
+__global__ void k_chunk_count(int nclu, int len, const int *__restrict__ tmpCnt,
+                              int *__restrict__ nch)
 {
     int I = blockIdx.x * blockDim.x + threadIdx.x;
-    if (I < nclu) nch[I] = (tmpCnt[I] + MDG_CHUNK - 1) / MDG_CHUNK;
+    if (I < nclu) nch[I] = (tmpCnt[I] + len - 1) / len;
 }
 
-__global__ void k_chunk_fill(int nclu, const int *__restrict__ cpOff, const int *__restrict__ chOff,
+__global__ void k_chunk_fill(int nclu, int len, const int *__restrict__ cpOff, const int *__restrict__ chOff,
                              int maxChunks, int2 *__restrict__ chunk, int *__restrict__ ctrl)
 {
     int I = blockIdx.x * blockDim.x + threadIdx.x;
     if (I >= nclu) return;
     for (int c = chOff[I]; c < chOff[I + 1]; c++) {
-        if (c < maxChunks) chunk[c] = make_int2(I, cpOff[I] + (c - chOff[I]) * MDG_CHUNK);
+        if (c < maxChunks) chunk[c] = make_int2(I, cpOff[I] + (c - chOff[I]) * len);
         else atomicOr(&ctrl[CTRL_LIST_OVF], 4);
     }
 }
@@ -938,6 +939,41 @@ static int sort_columns(mdg_ctx *ctx, const int *colOf, unsigned long long *keys
     return MDG_OK;
 }
 
+// Entries per work chunk.  Mixed: always MDG_CHUNK, over which the kernel sums
+// in FP32.  FP64: short enough for four chunks per SIMD (4,096 in all) where
+// the list is that long, at most 32 (the i-force reduction and its atomics come
+// once per chunk) and at least 2.
+static int chunk_len(const mdg_ctx *ctx, int entries)
+{
+    if (ctx->precision == MDG_MIXED) return MDG_CHUNK;
+    return std::min(std::max(entries / 4096, 2), MDG_CHUNK);
+}
+
+// Launch shapes of a step, by size (microseconds per step, 12 A cutoff and SPME
+// unless stated).
+// Fork order: the SPME branch is a chain of short kernels; started behind a pair
+// kernel that fills the chip it waits for it, started first it delays the pair
+// kernel by one launch.  SPME first against pair first:
+//   FP64  648 atoms 122 : 130, 3,000 142 : 160, 9,000 215 : 224, 24,000 355 : 351;
+//   mixed 3,000 126 : 135, 18,000 173 : 178, 30,000 199 : 193.
+// Pair grid: 1,024 blocks leave wave slots beside them; with more chunks than
+// that the last wave of long blocks costs more.  More blocks against 1,024:
+//   FP64  9,000 atoms 207 (2,048) : 215, 24,000 351 (2,048) : 375;
+//   mixed 18,000 179 (2,048) : 173, 30,000 199 : 193, 90,000 391 (4,096) : 400,
+//   192,000 744 (4,096) : 770; 256 replicas 881 (16,384) : 956.
+static void default_launch(mdg_ctx *ctx)
+{
+    if (ctx->tune.set) return;
+    const int n = ctx->n;
+    if (ctx->precision == MDG_MIXED) {
+        ctx->tune.spmeFirst = !ctx->bt && n <= 20000;
+        ctx->tune.pairBlocks = n <= 50000 ? 1024 : (ctx->bt ? 16384 : 4096);
+    } else {
+        ctx->tune.spmeFirst = !ctx->bt && n <= 12000;
+        ctx->tune.pairBlocks = n <= 6000 ? 1024 : 2048;
+    }
+}
+
 // Pair-count scan, list compaction and work chunks, shared by both
 // builders (C.tmpCnt / tmpJ / tmpMask filled by the pair search).  The
 // first call sizes the list from its own count with headroom.
@@ -956,7 +992,9 @@ static int compact_cluster_list(mdg_ctx *ctx)
         HIPCHK(hipMalloc(&C.cpJ, C.cap * sizeof(int)));
         HIPCHK(hipMalloc(&C.cpI, C.cap * sizeof(int)));
         HIPCHK(hipMalloc(&C.cpMask, C.cap * sizeof(unsigned long long)));
-        C.maxChunks = (int)(C.cap / MDG_CHUNK) + nclu + 64;
+        C.chunkLen = chunk_len(ctx, total);
+        default_launch(ctx);
+        C.maxChunks = (int)(C.cap / C.chunkLen) + nclu + 64;
         HIPCHK(hipMalloc(&C.chunk, (size_t)C.maxChunks * sizeof(int2)));
         HIPCHK(hipMalloc(&C.chOff, (nclu + 1) * sizeof(int)));
         if (ctx->precision == MDG_MIXED) {
@@ -980,11 +1018,11 @@ static int compact_cluster_list(mdg_ctx *ctx)
     // per-I chunk counts reuse tmpCnt's space after the compaction
     int *nch = C.sortTmp;   // n ints, free again after the column sort (n >= nclu)
     hipLaunchKernelGGL(k_chunk_count, dim3(nblk(nclu, 256)), dim3(256), 0, ctx->stream, nclu,
-                       C.tmpCnt, nch);
+                       C.chunkLen, C.tmpCnt, nch);
     LAUNCHCHK();
     RETCHK(mdg_scan_int(ctx, nch, C.chOff, nclu));
     hipLaunchKernelGGL(k_chunk_fill, dim3(nblk(nclu, 256)), dim3(256), 0, ctx->stream, nclu,
-                       C.cpOff, C.chOff, C.maxChunks, C.chunk, ctx->ctrl);
+                       C.chunkLen, C.cpOff, C.chOff, C.maxChunks, C.chunk, ctx->ctrl);
     LAUNCHCHK();
     return MDG_OK;
 }

@@ -63,21 +63,26 @@ __device__ constexpr double mdg_erfcx_c[MDG_ERFCX_N] = {
     -1.955135883083941e-09,
     -2.6231073623858514e-09};
 
-// erfc(x) for x >= 0, and ez = exp(-x^2).  The exponential's argument keeps
-// the rounding error of x^2 (its low part from an fma), without which the
-// relative error would grow as x^2.  Against 113-bit values over x in [0, 6]:
-// erfc within 7.1e-16 (the C library's: 6.7e-16), ez within 2.2e-16.
+// erfc(x) = exp(-x^2) p(y) / (1 + 2x) for x >= 0, and ez = exp(-x^2).  The
+// rounding errors of x^2, of 1/(1 + 2x) and of their product are kept (each
+// from one fma) and added with the last one, and y = (x - 3.75)/(x + 3.75) is
+// formed as 2x/(x + 3.75) - 1, which is exact enough where p is steep.
+// Against 113-bit values over x in [0, 6]: within 4.2e-16, rms 1.1e-16
+// (erfc() of the device library: 4.2e-16, 1.0e-16); ez within 2.2e-16.
 __device__ __forceinline__ double mdg_erfc64(double x, double &ez)
 {
     const double e = x * x, lo = __builtin_fma(x, x, -e);
-    double g = exp(-e);
-    g = __builtin_fma(-g, lo, g);
-    ez = g;
-    const double a = x + 3.75, b = __builtin_fma(2.0, x, 1.0);
+    const double g = exp(-e);
+    ez = __builtin_fma(-g, lo, g);
+    const double a = x + 3.75, x2 = x + x, b = x2 + 1.0;
     const double inv = mdg_rcp64(a * b);
-    const double y = ((x - 3.75) * b) * inv;
+    const double y = __builtin_fma(x2, b * inv, -1.0), r = a * inv;
     double p = mdg_erfcx_c[MDG_ERFCX_N - 1];
 #pragma unroll
     for (int k = MDG_ERFCX_N - 2; k >= 0; k--) p = __builtin_fma(p, y, mdg_erfcx_c[k]);
-    return (p * (a * inv)) * g;
+    const double bl = x2 - (b - 1.0);
+    const double c = __builtin_fma(-bl, r, __builtin_fma(-b, r, 1.0));
+    const double w = g * r;
+    const double wl = __builtin_fma(w, c - lo, __builtin_fma(g, r, -w));
+    return __builtin_fma(w, p, wl * p);
 }

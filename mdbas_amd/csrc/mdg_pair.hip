@@ -395,6 +395,7 @@ struct ClusterArgs {
     int maxChunks;                   // chunk capacity (an overflowing build is flagged)
     int cap;                         // entry capacity of cpJ / cpMask
     const int2 *chunk;               // chunk -> (I, first entry)
+    int chunkLen;                    // entries per chunk (FP64 kernels; mixed: MDG_CHUNK)
     long long *fix, *fiy, *fiz;      // MIXED: int64 fixed-point slot forces
     double *fdx, *fdy, *fdz;         // FP64: slot forces
     double *part;                    // per block: eDir, eVdw, virDir, virVdw, nIn
@@ -470,98 +471,157 @@ __device__ inline double dpp_sum8(double v)
     return v;
 }
 
+// dpp_rs8 in FP64: lanes a = 0, 2, 4 of each group end with the sums of x, y, z.
+template <int CTRL>
+__device__ __forceinline__ double dpp_movd(double v)
+{
+    const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xF, 0xF, true);
+    return __hiloint2double(hi, lo);
+}
+
+__device__ __forceinline__ double dpp_rs8d(double fx, double fy, double fz, int a)
+{
+    const bool hi = a >= 4;
+    double k0 = hi ? fz : fx, k1 = hi ? 0. : fy;
+    k0 += dpp_movd<0x141>(hi ? fx : fz);
+    k1 += dpp_movd<0x141>(hi ? fy : 0.);
+    const bool b1 = (a & 2) != 0;
+    double k = b1 ? k1 : k0;
+    k += dpp_movd<0x4E>(b1 ? k0 : k1);
+    k += dpp_movd<0xB1>(k);
+    return k;
+}
+
+// One entry's j slot b: position and parameters.
+struct Fp64J {
+    double x, y, z, q, e, g;
+};
+
+__device__ __forceinline__ Fp64J fp64_load(const ClusterArgs &A, int sj)
+{
+    return {A.sx[sj], A.sy[sj], A.sz[sj], A.sq[sj], A.seps[sj], A.ssig[sj]};
+}
+
+// Minimum image and r^2 as mdg_dist forms them, the image index rounded by
+// rint (see mx_ref_r2: the same for every pair inside the cutoff).
+__device__ __forceinline__ double fp64_dist(const MdgBox &b, double &dx, double &dy, double &dz)
+{
+#pragma clang fp contract(off)
+    if (b.type == 3) return mdg_dist(b, dx, dy, dz);
+    const double L1 = b.type == 1 ? b.a1 : b.b2, L2 = b.type == 1 ? b.a1 : b.c3;
+    const double i1 = b.type == 1 ? b.u1 : b.v2, i2 = b.type == 1 ? b.u1 : b.w3;
+    if (b.type != 0) {
+        dx -= b.a1 * rint(dx * b.u1);
+        dy -= L1 * rint(dy * i1);
+        dz -= L2 * rint(dz * i2);
+    }
+    return dx * dx + dy * dy + dz * dz;
+}
+
 // Lane mapping: a = lane & 7 is the i atom, b = lane >> 3 the j atom, so
 // each j-cluster pair's j-force sums run over 8 adjacent lanes (DPP) and
 // the i-force sums over lanes a, a+8, ..., a+56 happen once per chunk.
 // Mask bit 8 b + a (= the lane) marks the listed pair (I_a, J_b).  FP64
-// throughout.
+// throughout.  Entry, j cluster and mask are wave-uniform (scalar cache), and
+// the next entry's j slots are requested before the current one is computed.
+//
+// Bound by FP64 issue once there are enough wavefronts, and by one entry's
+// latency (about 1.7 us for a lone wavefront) when there are not: a small box
+// has few chunks of 32 entries, so its chunks are shorter (chunk_len).  Before,
+// with 32 entries a chunk, library sqrt / divide / erfc / exp and per-component
+// DPP sums: 648 atoms 47.7 us, now 8.4; 3,000 atoms 59 -> 43; 12,000 atoms
+// 185 -> 148.  The j atomics are a fifth of what is left.
 template <bool BATCH, int ELEC>
 __global__ void __launch_bounds__(256) k_pair_fp64(ClusterArgs A)
 {
     const int lane = threadIdx.x & 63;
     const int a = lane & 7, b = lane >> 3;
-    const int bit = lane;
     double e_acc[5] = {0, 0, 0, 0, 0};
-    const int nch = min(A.chOff[A.nclu], A.maxChunks);
-    for (int W = blockIdx.x * 4 + (threadIdx.x >> 6); W < nch; W += gridDim.x * 4) {
-        // chunk W: entries [e0, e1) of i-cluster I (at most MDG_CHUNK of them)
-        const int2 ch = A.chunk[W];
-        const int I = ch.x, e0 = ch.y, e1 = min(min(e0 + MDG_CHUNK, A.cpOff[I + 1]), A.cap);
+    const int nch = min(mdg_uload(A.chOff, A.nclu), A.maxChunks);
+    for (int W = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); W < nch;
+         W += gridDim.x * 4) {
+        // chunk W: entries [e0, e1) of i-cluster I
+        const long ch = mdg_uload((const long *)A.chunk, W);   // int2 (I, e0)
+        const int I = (int)(ch & 0xffffffffl), e0 = (int)(ch >> 32);
+        const int e1 = min(min(e0 + A.chunkLen, mdg_uload(A.cpOff, I + 1)), A.cap);
         if (e0 >= e1) {   // only after a flagged list overflow
             if (BATCH && lane < 5) A.chE[(long)W * 5 + lane] = 0.;
             continue;
         }
         // the box: the run's, or the replica's in a batch
-        const MdgBox &Bx = BATCH ? A.boxes[A.crep[I]] : A.B;
+        const MdgBox &Bx = BATCH ? A.boxes[mdg_uload(A.crep, I)] : A.B;
         const int si = I * MDG_CL + a;
-        const double xi = A.sx[si], yi = A.sy[si], zi = A.sz[si];
-        const double qid = A.sq[si], eid = A.seps[si], gid = A.ssig[si];
+        const Fp64J pi = fp64_load(A, si);
         double fxid = 0., fyid = 0., fzid = 0.;
         double ed = 0., ev = 0., vd = 0., vv = 0.;
         int nin = 0;
+        int J = mdg_uload(A.cpJ, e0);
+        unsigned long long m = mdg_uload(A.cpMask, e0);
+        Fp64J pj = fp64_load(A, J * MDG_CL + b);
         for (int e = e0; e < e1; e++) {
-            const int J = A.cpJ[e];
-            const unsigned long long m = A.cpMask[e];
-            const int sj = J * MDG_CL + b;
-            double dx = A.sx[sj] - xi, dy = A.sy[sj] - yi, dz = A.sz[sj] - zi;
-            const double r2 = mdg_dist(Bx, dx, dy, dz);
-            const bool inCut = ((m >> bit) & 1ull) && r2 <= A.P.cutOff2;
+            const int en = min(e + 1, e1 - 1);
+            const int Jn = mdg_uload(A.cpJ, en);
+            const unsigned long long mn = mdg_uload(A.cpMask, en);
+            const Fp64J pn = fp64_load(A, Jn * MDG_CL + b);
+            double dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+            const double r2 = fp64_dist(Bx, dx, dy, dz);
+            const unsigned long long inm = m & __builtin_amdgcn_ballot_w64(r2 <= A.P.cutOff2);
             // an entry with no pair inside the cutoff adds only exact zeros
-            if (__builtin_amdgcn_ballot_w64(inCut) == 0) continue;
-            double fjx = 0., fjy = 0., fjz = 0.;
-            if (inCut) {
-                const double r = sqrt(r2), rt = 1. / r;
-                double dEl = 0., dVw = 0., el = 0., evw = 0.;
-                if (ELEC == PAIR_EWALD)
-                    el = ewald_dir64(A.P.alpha, A.P.chargeConst * qid * A.sq[sj], r, rt, dEl);
-                else if (ELEC != PAIR_NONE)
-                    el = coulomb64(A.P, ELEC, qid * A.sq[sj], r2, rt, dEl);
-                if (A.P.vdwOn)
-                    evw = vdw_switch64(A.P, eid * A.seps[sj], gid + A.ssig[sj], r2, rt, dVw);
-                const double fs = dEl + dVw;
-                fjx = fs * dx * rt;
-                fjy = fs * dy * rt;
-                fjz = fs * dz * rt;
-                ed += el;
-                ev += evw;
-                vd += dEl * r;
-                vv += dVw * r;
-                nin++;
+            if (inm != 0) {
+                double fjx = 0., fjy = 0., fjz = 0.;
+                nin += __builtin_popcountll(inm);
+                if (__builtin_amdgcn_inverse_ballot_w64(inm)) {
+                    double r;
+                    const double rt = mdg_rsqrt64(r2, r);
+                    double dEl = 0., dVw = 0., el = 0., evw = 0.;
+                    if (ELEC == PAIR_EWALD)
+                        el = ewald_dir64(A.P.alpha, A.P.chargeConst * pi.q * pj.q, r, rt, dEl);
+                    else if (ELEC != PAIR_NONE)
+                        el = coulomb64(A.P, ELEC, pi.q * pj.q, r2, rt, dEl);
+                    if (A.P.vdwOn)
+                        evw = vdw_switch64(A.P, pi.e * pj.e, pi.g + pj.g, r2, rt, dVw);
+                    const double fs = (dEl + dVw) * rt;
+                    fjx = fs * dx;
+                    fjy = fs * dy;
+                    fjz = fs * dz;
+                    ed += el;
+                    ev += evw;
+                    vd += dEl * r;
+                    vv += dVw * r;
+                    fxid += fjx;
+                    fyid += fjy;
+                    fzid += fjz;
+                }
+                const double k = dpp_rs8d(fjx, fjy, fjz, a);
+                const int sj = J * MDG_CL + b;
+                if ((a & 1) == 0 && a < 6 && k != 0.)
+                    atomicAdd(a == 0 ? &A.fdx[sj] : (a == 2 ? &A.fdy[sj] : &A.fdz[sj]), -k);
             }
-            fxid += fjx;
-            fyid += fjy;
-            fzid += fjz;
-            fjx = dpp_sum8(fjx);
-            fjy = dpp_sum8(fjy);
-            fjz = dpp_sum8(fjz);
-            if (a == 0) {
-                if (fjx != 0.) atomicAdd(&A.fdx[sj], -fjx);
-                if (fjy != 0.) atomicAdd(&A.fdy[sj], -fjy);
-                if (fjz != 0.) atomicAdd(&A.fdz[sj], -fjz);
-            }
+            J = Jn;
+            m = mn;
+            pj = pn;
         }
         for (int o = 8; o < 64; o <<= 1) {
             fxid += __shfl_xor(fxid, o, 64);
             fyid += __shfl_xor(fyid, o, 64);
             fzid += __shfl_xor(fzid, o, 64);
         }
-        if (b == 0) {
-            atomicAdd(&A.fdx[si], fxid);
-            atomicAdd(&A.fdy[si], fyid);
-            atomicAdd(&A.fdz[si], fzid);
-        }
+        if (b < 3)
+            atomicAdd(b == 0 ? &A.fdx[si] : (b == 1 ? &A.fdy[si] : &A.fdz[si]),
+                      b == 0 ? fxid : (b == 1 ? fyid : fzid));
         if (BATCH) {
             // energies per chunk, summed per replica later (a replica's
             // chunks are contiguous)
             const double c[5] = {mdg_wave_sum(ed), mdg_wave_sum(ev), mdg_wave_sum(vd),
-                                 mdg_wave_sum(vv), mdg_wave_sum((double)nin)};
+                                 mdg_wave_sum(vv), (double)nin};
             if (lane < 5) A.chE[(long)W * 5 + lane] = c[lane];
         } else {
             e_acc[0] += ed;
             e_acc[1] += ev;
             e_acc[2] += vd;
             e_acc[3] += vv;
-            e_acc[4] += nin;
+            e_acc[4] += lane == 0 ? (double)nin : 0.;
         }
     }
     if (!BATCH) mdg_block_partials<5>(e_acc, A.part);
@@ -1165,6 +1225,7 @@ static ClusterArgs cluster_args(mdg_ctx *ctx)
     A.chOff = C.chOff;
     A.chunk = C.chunk;
     A.maxChunks = C.maxChunks;
+    A.chunkLen = C.chunkLen;
     A.cap = (int)C.cap;
     A.fix = ctx->fix;
     A.fiy = ctx->fiy;
@@ -1391,7 +1452,7 @@ __global__ void __launch_bounds__(256) k_adj_cluster(ClusterArgs A)
     const int nch = min(A.chOff[A.nclu], A.maxChunks);
     for (int W = blockIdx.x * 4 + (threadIdx.x >> 6); W < nch; W += gridDim.x * 4) {
         const int2 ch = A.chunk[W];
-        const int I = ch.x, e0 = ch.y, e1 = min(min(e0 + MDG_CHUNK, A.cpOff[I + 1]), A.cap);
+        const int I = ch.x, e0 = ch.y, e1 = min(min(e0 + A.chunkLen, A.cpOff[I + 1]), A.cap);
         const int si = I * MDG_CL + a;
         const double xi = A.sx[si], yi = A.sy[si], zi = A.sz[si];
         const double qi = A.sq[si], ei = A.seps[si], gi = A.ssig[si];
@@ -1497,7 +1558,7 @@ __global__ void __launch_bounds__(256) k_hvp_cluster(ClusterArgs A, HvpSlots H)
     const double C = A.P.chargeConst, al = A.P.alpha;
     for (int W = blockIdx.x * 4 + (threadIdx.x >> 6); W < nch; W += gridDim.x * 4) {
         const int2 ch = A.chunk[W];
-        const int I = ch.x, e0 = ch.y, e1 = min(min(e0 + MDG_CHUNK, A.cpOff[I + 1]), A.cap);
+        const int I = ch.x, e0 = ch.y, e1 = min(min(e0 + A.chunkLen, A.cpOff[I + 1]), A.cap);
         const int si = I * MDG_CL + a;
         const double xi = A.sx[si], yi = A.sy[si], zi = A.sz[si];
         const double qi = A.sq[si], ei = A.seps[si], gi = A.ssig[si];

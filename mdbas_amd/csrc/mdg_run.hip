@@ -634,6 +634,7 @@ extern "C" int mdg_set_prune(mdg_ctx *ctx, double skin)
     }
     if (skin > ctx->P.delr) skin = ctx->P.delr;
     ctx->pruneSkin = skin;
+    ctx->pruneSet = true;
     mdg_invalidate_graphs(ctx);
     return MDG_OK;
 }
@@ -671,6 +672,7 @@ extern "C" int mdg_set_launch(mdg_ctx *ctx, const int in[4])
     ctx->tune.pairBlocks = in[1];
     ctx->tune.spmeFirst = in[2];
     ctx->tune.spmePrio = in[3];
+    ctx->tune.set = true;
     mdg_invalidate_graphs(ctx);
     return MDG_OK;
 }
@@ -1009,8 +1011,9 @@ static int time_steps(mdg_ctx *ctx, const double *state, int nsteps, float &ms)
 // Picks the launch shapes of this system on this GPU by timing whole steps
 // (graph-replayed, as mdg_run_steps runs them): the three-site SHAKE
 // spread, the pair kernel's grid cap, the branch order at the fork, the
-// SPME kernels' wave priority, and (when pruning is on) the pruned list
-// against the full one, one after the other with the rest held.  The uploaded state is restored afterwards and
+// SPME kernels' wave priority, and (where the boxes have room and the caller
+// did not switch it off) the pruned list against the full one, one after the
+// other with the rest held.  The uploaded state is restored afterwards and
 // the initial energy recomputed.  out (may be NULL): the chosen spread and
 // pair-grid cap (mdg_get_launch has all of them).
 extern "C" int mdg_autotune(mdg_ctx *ctx, int nsteps, int out[2])
@@ -1053,10 +1056,12 @@ extern "C" int mdg_autotune(mdg_ctx *ctx, int nsteps, int out[2])
         sweep(&ctx->tune.spmeFirst, {0, 1});
         sweep(&ctx->tune.spmePrio, {0, 1, 2});
     }
-    if (ctx->pruneSkin > 0. && st == MDG_OK) {
+    // the distance in use, or the usual one unless the caller switched it off
+    const double skin = ctx->pruneSet ? ctx->pruneSkin : mdg_prune_candidate(ctx);
+    if (skin > 0. && st == MDG_OK) {
         // the pruned list, or the full list every step (no prune kernel)
-        const double skin = ctx->pruneSkin;
         float msOn = 0.f, msOff = 0.f;
+        ctx->pruneSkin = skin;
         mdg_invalidate_graphs(ctx);
         st = time_steps(ctx, state, nsteps, msOn);
         ctx->pruneSkin = 0.;
@@ -1064,6 +1069,7 @@ extern "C" int mdg_autotune(mdg_ctx *ctx, int nsteps, int out[2])
         if (st == MDG_OK) st = time_steps(ctx, state, nsteps, msOff);
         ctx->pruneSkin = (st == MDG_OK && msOff < msOn) ? 0. : skin;
     }
+    ctx->tune.set = true;
     mdg_invalidate_graphs(ctx);
     for (int k = 0; k < 6 && st == MDG_OK; k++)
         if (hipMemcpyAsync(d[k], state + k * n, n * sizeof(double), hipMemcpyDeviceToDevice,
