@@ -186,6 +186,22 @@ struct MdgTune {
     bool set = false;            // chosen by mdg_set_launch or mdg_autotune: no default by size
 };
 
+// One axis of the FP64 mesh convolution (mdg_conv64.hip): its length and the
+// passes' radices, with the multipliers (2^32 / d + 1) that divide by the
+// transformed length so far and by the butterflies of a transform.
+#define CONV_PASSES 8
+struct ConvAxis {
+    int n = 0, np = 0;
+    int r[CONV_PASSES] = {};
+    unsigned mL[CONV_PASSES] = {}, mT[CONV_PASSES] = {};
+};
+
+struct ConvPlan {
+    ConvAxis x, y, z;            // z: half the real length
+    int mh = 0;
+    unsigned mMh = 0, mNz = 0, mCols = 0;
+};
+
 struct mdg_ctx {
     int precision = MDG_FP64;
     int n = 0;
@@ -302,6 +318,9 @@ struct mdg_ctx {
     double *theta = nullptr;     // [m1][m2][mh]
     float *theta32 = nullptr;
     double *grid64 = nullptr;    // real mesh (FP64)
+    ConvPlan conv;
+    bool convOn = false;         // FP64 meshes take mdg_conv64, else rocFFT
+    void *convTw = nullptr;      // its roots of unity, x | y | z
     double *cgrid64 = nullptr;   // complex half spectrum (FP64, interleaved)
     float *grid32 = nullptr;
     float *cgrid32 = nullptr;
@@ -630,7 +649,16 @@ int mdg_spme_device(mdg_ctx *ctx);   // device-resident: frx.. per atom, partial
 int mdg_spme_fork(mdg_ctx *ctx);   // marks the point stream2's work starts from
 int mdg_spme_on(mdg_ctx *ctx, int (*fn)(mdg_ctx *));   // runs fn's launches on stream2 from it
 // blocks (= partial rows) of the SPME influence kernel over H half-spectrum points
+int mdg_conv64_setup(mdg_ctx *ctx);   // mdg_conv64.hip
+int mdg_conv64_rows(const mdg_ctx *ctx);
+int mdg_conv64(mdg_ctx *ctx, double *grid, double *part, bool clearBins);
 inline int mdg_infl_blocks(long H) { return (int)std::min<long>(nblk(H, 256), 256); }
+// rows of the reciprocal energy and stress partials
+inline int mdg_infl_rows(const mdg_ctx *ctx, bool fp64)
+{
+    return fp64 && ctx->convOn ? mdg_conv64_rows(ctx)
+                               : mdg_infl_blocks((long)ctx->m1 * ctx->m2 * ctx->mh);
+}
 int mdg_gather_blocks(const mdg_ctx *ctx);   // block partials of the reciprocal forces
 int mdg_spme_pot(mdg_ctx *ctx, double *pot);   // FP64 dE_rec/dq per atom
 int mdg_adj_pair(mdg_ctx *ctx);      // real-space dE/d(q, eps, sig) into fdx/fdy/fdz slots

@@ -234,7 +234,7 @@ RecArgs mdg_rec_args(mdg_ctx *ctx, int nbKin, int nGrpVir, int nbExcl)
     R.recCap = ctx->recCap;
     R.nbPair = mdg_pair_blocks(ctx);
     R.nbExcl = nbExcl;
-    R.nbInfl = ew ? mdg_infl_blocks((long)ctx->m1 * ctx->m2 * ctx->mh) : 0;
+    R.nbInfl = ew ? mdg_infl_rows(ctx, ctx->precision != MDG_MIXED) : 0;
     R.nbKin = nbKin;
     R.nGrpVir = nGrpVir;
     R.pPair = ctx->epart + PART_PAIR;

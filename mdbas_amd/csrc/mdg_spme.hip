@@ -515,13 +515,101 @@ __device__ inline int spme_tile_bins(int X0, int m, int *bins)
 {
     int nb = 0, last = -1;
     for (int d = 0; d < SPME_TILE + P - 1; d++) {
-        const int top = (X0 + d) % m, b = top / SPME_BIN;
+        const int t = X0 + d, top = t >= m ? t - m : t, b = top / SPME_BIN;
         if (b != last) {
             bins[nb++] = b;
             last = b;
         }
     }
     return nb;
+}
+
+// A tile's spreading, in rounds of one atom per thread.  First each thread takes
+// one candidate of the tile's buckets, drops it if none of its P^3 points lies in
+// the tile (about half do not), and leaves its splines in LDS; then the block
+// adds, P^2 lanes per atom.  One thread per atom doing all P^3 points, as before,
+// left most of a block idle (a tile of a small mesh has 60 candidates for 256
+// threads) behind a chain of 64 dependent range checks.  Bound by that latency on
+// small meshes: 14 us -> 11 at 20^3 and 9.5 at 48^3 (FP64); on large ones by the
+// LDS adds and the pair kernel beside it.
+//
+// One round's atoms of a tile: per atom q times the splines along index 1, the
+// splines along 2 and 3, and where each of the 3 P mesh rows lies in the tile
+// (four bits a row, 15 outside it).  The odd row keeps the banks apart.
+template <int P, typename T>
+struct SpreadLds {
+    T b[256][3 * P + 1];
+    unsigned row[3][256];
+    int cnt;
+};
+
+// Adds nh atoms' products into the tile: one lane per atom and (j, k), looping
+// over i, so neighbouring lanes add to neighbouring points.
+template <int P, typename T>
+__device__ __forceinline__ void spread_add(const SpreadLds<P, T> &S, int nh,
+                                           unsigned long long *acc)
+{
+    constexpr int TL = SPME_TILE;
+    for (int w = threadIdx.x; w < nh * P * P; w += blockDim.x) {
+        const int c = w / (P * P), jk = w - c * (P * P), j = jk / P, k = jk - j * P;
+        const unsigned ly = (S.row[1][c] >> (4 * j)) & 15u, lz = (S.row[2][c] >> (4 * k)) & 15u;
+        if (ly == 15u || lz == 15u) continue;
+        const unsigned r0 = S.row[0][c], o = ly * TL + lz;
+        const T bj = S.b[c][P + j], bk = S.b[c][2 * P + k];
+#pragma unroll
+        for (int i = 0; i < P; i++) {
+#pragma clang fp contract(off)
+            const unsigned lx = (r0 >> (4 * i)) & 15u;
+            if (lx == 15u) continue;
+            const T v = S.b[c][i] * bj * bk;
+            if (sizeof(T) == 8)
+                atomicAdd(reinterpret_cast<double *>(acc) + lx * TL * TL + o, (double)v);
+            else
+                atomicAdd(&acc[lx * TL * TL + o],
+                          (unsigned long long)__double2ll_rn((double)v * MDG_QSCALE));
+        }
+    }
+}
+
+// The tile rows of an atom's P mesh indices below base along one dimension.
+template <int P>
+__device__ __forceinline__ unsigned spread_rows(int base, int m, int X0, bool &hit)
+{
+    unsigned r = 0;
+    bool any = false;
+#pragma unroll
+    for (int i = 0; i < P; i++) {
+        const int l = wrap_index(base - i, m) - X0;
+        const bool in = l >= 0 && l < SPME_TILE;
+        r |= (in ? (unsigned)l : 15u) << (4 * i);
+        any |= in;
+    }
+    hit &= any;
+    return r;
+}
+
+// Appends the lane's atom (valid: it has one) if it touches the tile.
+template <int P, typename T>
+__device__ __forceinline__ void spread_put(SpreadLds<P, T> &S, bool valid, T ql, const T *b1,
+                                           const T *b2, const T *b3, unsigned r1, unsigned r2,
+                                           unsigned r3)
+{
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(valid);
+    if (m == 0) return;
+    const int lane = threadIdx.x & 63;
+    int at = 0;
+    if (lane == 0) at = atomicAdd(&S.cnt, __builtin_popcountll(m));
+    at = __builtin_amdgcn_readfirstlane(at) + __builtin_popcountll(m & ((1ull << lane) - 1));
+    if (!valid) return;
+#pragma unroll
+    for (int i = 0; i < P; i++) {
+        S.b[at][i] = ql * b1[i];
+        S.b[at][P + i] = b2[i];
+        S.b[at][2 * P + i] = b3[i];
+    }
+    S.row[0][at] = r1;
+    S.row[1][at] = r2;
+    S.row[2][at] = r3;
 }
 
 // F64: the FP64 mesh of the FP64 path.  Each bucketed atom's splines are
@@ -585,10 +673,17 @@ k_spme_spread_tiles(MdgParams Pm, MdgBox B, int nty, int ntz, int nby, int nbz,
         if (lane == 0) off[nbt] = run;
     }
     __syncthreads();
+    typedef typename std::conditional<F64, double, float>::type TS;
+    __shared__ SpreadLds<P, TS> S;
     const int ncand = off[nbt], nout = binNOut[0];
     for (int c0 = 0; c0 < ncand + nout; c0 += blockDim.x) {
         const int c = c0 + threadIdx.x;
-        if (c < ncand + nout) {
+        if (threadIdx.x == 0) S.cnt = 0;
+        __syncthreads();
+        bool hit = c < ncand + nout;
+        TS b[3][P] = {}, ql = 0;
+        unsigned row[3] = {0, 0, 0};
+        if (hit) {
             int l;
             if (c < ncand) {
                 int lo = 0, hi = nbt;   // off[lo] <= c < off[hi]
@@ -601,61 +696,37 @@ k_spme_spread_tiles(MdgParams Pm, MdgBox B, int nty, int ntz, int nby, int nbz,
             } else {
                 l = binOut[c - ncand];
             }
+            int base[3];
+            double s[3];
             if (F64) {
-#pragma clang fp contract(off)
-                double s1, s2, s3;
-                scaled_coords(B, m1, m2, m3, x[l], y[l], z[l], s1, s2, s3);
-                double b1[P], b2[P], b3[P], d[P];
-                bspline_fix<double, P>(s1, b1, d);
-                bspline_fix<double, P>(s2, b2, d);
-                bspline_fix<double, P>(s3, b3, d);
-                const int i1 = (int)s1, i2 = (int)s2, i3 = (int)s3;
-                const double ql = q[l];
-                double *acc64 = reinterpret_cast<double *>(acc);
-#pragma unroll
-                for (int i = 0; i < P; i++) {
-                    const int lx = wrap_index(i1 - i, m1) - X0;
-                    if (lx < 0 || lx >= T) continue;
-                    const double qa = ql * b1[i];
-#pragma unroll
-                    for (int j = 0; j < P; j++) {
-                        const int ly = wrap_index(i2 - j, m2) - Y0;
-                        if (ly < 0 || ly >= T) continue;
-                        const double qb = qa * b2[j];
-#pragma unroll
-                        for (int k = 0; k < P; k++) {
-                            const int lz = wrap_index(i3 - k, m3) - Z0;
-                            if (lz < 0 || lz >= T) continue;
-                            atomicAdd(&acc64[(lx * T + ly) * T + lz], qb * b3[k]);
-                        }
-                    }
-                }
+                scaled_coords(B, m1, m2, m3, x[l], y[l], z[l], s[0], s[1], s[2]);
+                for (int d = 0; d < 3; d++) base[d] = (int)s[d];
             } else {
-                SplineAtom<P> S;
-                spline_load<P>(splI, splB, nullptr, Pm.n, l, false, S);
-                const float ql = (float)q[l];
-#pragma unroll
-                for (int i = 0; i < P; i++) {
-                    const int lx = wrap_index(S.base[0] - i, m1) - X0;
-                    if (lx < 0 || lx >= T) continue;
-                    const float qa = ql * S.b[0][i];
-#pragma unroll
-                    for (int j = 0; j < P; j++) {
-                        const int ly = wrap_index(S.base[1] - j, m2) - Y0;
-                        if (ly < 0 || ly >= T) continue;
-                        const float qb = qa * S.b[1][j];
-#pragma unroll
-                        for (int k = 0; k < P; k++) {
-                            const int lz = wrap_index(S.base[2] - k, m3) - Z0;
-                            if (lz < 0 || lz >= T) continue;
-                            const long long v =
-                                __double2ll_rn((double)(qb * S.b[2][k]) * MDG_QSCALE);
-                            atomicAdd(&acc[(lx * T + ly) * T + lz], (unsigned long long)v);
-                        }
-                    }
+                const int4 bi = splI[l];
+                base[0] = bi.x;
+                base[1] = bi.y;
+                base[2] = bi.z;
+            }
+            row[0] = spread_rows<P>(base[0], m1, X0, hit);
+            row[1] = spread_rows<P>(base[1], m2, Y0, hit);
+            row[2] = spread_rows<P>(base[2], m3, Z0, hit);
+            if (hit) {
+                ql = (TS)q[l];
+                if constexpr (F64) {
+                    double d[P];
+                    for (int k = 0; k < 3; k++) bspline_fix<double, P>(s[k], b[k], d);
+                } else {
+                    SplineAtom<P> A;
+                    spline_load<P>(splI, splB, nullptr, Pm.n, l, false, A);
+                    for (int k = 0; k < 3; k++)
+                        for (int i = 0; i < P; i++) b[k][i] = A.b[k][i];
                 }
             }
         }
+        spread_put<P, TS>(S, hit, ql, b[0], b[1], b[2], row[0], row[1], row[2]);
+        __syncthreads();
+        spread_add<P, TS>(S, S.cnt, acc);
+        __syncthreads();
     }
     __syncthreads();
     for (int i = threadIdx.x; i < T * T * T; i += blockDim.x) {
@@ -730,7 +801,8 @@ static int spread_binned_p(mdg_ctx *ctx)
                        ctx->z, ctx->q, ctx->binCnt, ctx->binBucket, ctx->binOut, ctx->binNOut,
                        ctx->splI, ctx->splB, ctx->grid32, ctx->grid64);
     LAUNCHCHK();
-    if (F64) {
+    // (the convolution's first kernel does it where it runs)
+    if (F64 && !ctx->convOn) {
         const long nb = (long)ctx->nbx * ctx->nby * ctx->nbz;
         hipLaunchKernelGGL(k_bin_clear, dim3((int)std::min<long>(nblk(nb, 256), 1024)), dim3(256),
                            0, ctx->stream, nb, ctx->binCnt, ctx->binNOut);
@@ -1090,7 +1162,8 @@ int mdg_spme_setup(mdg_ctx *ctx)
         return MDG_EHIP;
     }
     rocfft_execution_info_set_stream(ctx->info, ctx->stream);
-    RETCHK(make_plans(ctx, true, &ctx->fwd, &ctx->bwd));
+    RETCHK(mdg_conv64_setup(ctx));
+    if (!ctx->convOn) RETCHK(make_plans(ctx, true, &ctx->fwd, &ctx->bwd));
     if (ctx->precision == MDG_MIXED) {
         HIPCHK(hipMalloc(&ctx->grid32, G * sizeof(float)));
         HIPCHK(hipMalloc(&ctx->cgrid32, 2 * H * sizeof(float)));
@@ -1109,8 +1182,47 @@ int mdg_spme_free(mdg_ctx *ctx)
     if (ctx->fwd32) rocfft_plan_destroy(ctx->fwd32);
     if (ctx->bwd32) rocfft_plan_destroy(ctx->bwd32);
     if (ctx->info) rocfft_execution_info_destroy(ctx->info);
+    if (ctx->convTw) (void)hipFree(ctx->convTw);
+    ctx->convTw = nullptr;
+    ctx->convOn = false;
     ctx->fwd = ctx->bwd = ctx->fwd32 = ctx->bwd32 = nullptr;
     ctx->info = nullptr;
+    return MDG_OK;
+}
+
+// cg *= theta on the half spectrum (the influence function of spme.c:505-583).
+__global__ void k_theta_mul(long H, const double *__restrict__ theta, double *cg)
+{
+    const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (g >= H) return;
+    cg[2 * g] *= theta[g];
+    cg[2 * g + 1] *= theta[g];
+}
+
+// grid <- theta * grid through rocFFT; part (may be null): the energy and
+// stress partials of mdg_infl_blocks rows.  For meshes mdg_conv64 leaves out.
+static int fft_conv64(mdg_ctx *ctx, double *grid, double *part)
+{
+    const int m1 = ctx->m1, m2 = ctx->m2, m3 = ctx->m3, mh = ctx->mh;
+    const long H = (long)m1 * m2 * mh;
+    void *in[1] = {grid}, *out[1] = {ctx->cgrid64};
+    if (rocfft_execute(ctx->fwd, in, out, ctx->info) != rocfft_status_success) {
+        ctx->err = "rocfft_execute (forward) failed";
+        return MDG_EHIP;
+    }
+    if (part)
+        hipLaunchKernelGGL(k_spme_influence<double>, dim3(mdg_infl_blocks(H)), dim3(256), 0,
+                           ctx->stream, ctx->B, m1, m2, m3, mh,
+                           -0.25 / (ctx->P.alpha * ctx->P.alpha), ctx->theta, ctx->cgrid64, part);
+    else
+        hipLaunchKernelGGL(k_theta_mul, dim3(nblk(H, 256)), dim3(256), 0, ctx->stream, H,
+                           ctx->theta, ctx->cgrid64);
+    LAUNCHCHK();
+    void *in2[1] = {ctx->cgrid64}, *out2[1] = {grid};
+    if (rocfft_execute(ctx->bwd, in2, out2, ctx->info) != rocfft_status_success) {
+        ctx->err = "rocfft_execute (inverse) failed";
+        return MDG_EHIP;
+    }
     return MDG_OK;
 }
 
@@ -1158,20 +1270,10 @@ static int spme_run(mdg_ctx *ctx, bool mixed, double *partInfl, double *partGath
             launch_spread<false>(ctx, ctx->grid64, nullptr);
             LAUNCHCHK();
         }
-        void *in[1] = {ctx->grid64}, *out[1] = {ctx->cgrid64};
-        if (rocfft_execute(ctx->fwd, in, out, ctx->info) != rocfft_status_success) {
-            ctx->err = "rocfft_execute (forward) failed";
-            return MDG_EHIP;
-        }
-        hipLaunchKernelGGL(k_spme_influence<double>, dim3(mdg_infl_blocks(H)), dim3(256), 0,
-                           ctx->stream, ctx->B, m1, m2, m3, mh, rAlpha2, ctx->theta, ctx->cgrid64,
-                           partInfl);
-        LAUNCHCHK();
-        void *in2[1] = {ctx->cgrid64}, *out2[1] = {ctx->grid64};
-        if (rocfft_execute(ctx->bwd, in2, out2, ctx->info) != rocfft_status_success) {
-            ctx->err = "rocfft_execute (inverse) failed";
-            return MDG_EHIP;
-        }
+        if (ctx->convOn)
+            RETCHK(mdg_conv64(ctx, ctx->grid64, partInfl, spme_binned(ctx)));
+        else
+            RETCHK(fft_conv64(ctx, ctx->grid64, partInfl));
         launch_gather<false>(ctx, (const double *)ctx->grid64, fact1, (double *)frx,
                              (double *)fry, (double *)frz, partGather);
         LAUNCHCHK();
@@ -1229,10 +1331,9 @@ __global__ void k_sub_mean(int n, double *fx, double *fy, double *fz, const doub
 int mdg_spme64(mdg_ctx *ctx, double *fx, double *fy, double *fz, double eout[8])
 {
     const int n = ctx->n;
-    const long H = (long)ctx->m1 * ctx->m2 * ctx->mh;
     RETCHK(spme_run(ctx, false, ctx->epart + PART_INFL, ctx->epart + PART_GATHER, ctx->frx64,
                     ctx->fry64, ctx->frz64));
-    RETCHK(mdg_reduce_partials(ctx, ctx->epart + PART_INFL, mdg_infl_blocks(H), 7,
+    RETCHK(mdg_reduce_partials(ctx, ctx->epart + PART_INFL, mdg_infl_rows(ctx, true), 7,
                                ctx->scal + S_EREC));
     hipLaunchKernelGGL(k_add_rec, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, n, fx, fy, fz,
                        ctx->frx64, ctx->fry64, ctx->frz64, ctx->epart + PART_MISC);
@@ -1342,15 +1443,6 @@ k_hvp_spread(MdgParams P, MdgBox B, int n, const double *__restrict__ x,
     }
 }
 
-// cg *= theta on the half spectrum (the influence function of spme.c:505-583).
-__global__ void k_theta_mul(long H, const double *__restrict__ theta, double *cg)
-{
-    const long g = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (g >= H) return;
-    cg[2 * g] *= theta[g];
-    cg[2 * g + 1] *= theta[g];
-}
-
 // Per atom, with phi = theta * Q (grid) and phi_u = theta * Q_u (gridU),
 // f2 = 2 (2 pi / V) C:
 //   hu_l += f2 q_l sum_g [phi (Hess W_l) u_l + phi_u grad W_l]
@@ -1428,19 +1520,10 @@ int mdg_spme_hvp(mdg_ctx *ctx, const double *u, const double s[3], double *hu, d
     hipLaunchKernelGGL(k_hvp_spread, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, ctx->P, ctx->B,
                        n, ctx->x, ctx->y, ctx->z, ctx->q, u, sv, ctx->gridU);
     LAUNCHCHK();
-    void *in[1] = {ctx->gridU}, *out[1] = {ctx->cgrid64};
-    if (rocfft_execute(ctx->fwd, in, out, ctx->info) != rocfft_status_success) {
-        ctx->err = "rocfft_execute (forward) failed";
-        return MDG_EHIP;
-    }
-    hipLaunchKernelGGL(k_theta_mul, dim3(nblk(H, 256)), dim3(256), 0, ctx->stream, H, ctx->theta,
-                       ctx->cgrid64);
-    LAUNCHCHK();
-    void *in2[1] = {ctx->cgrid64}, *out2[1] = {ctx->gridU};
-    if (rocfft_execute(ctx->bwd, in2, out2, ctx->info) != rocfft_status_success) {
-        ctx->err = "rocfft_execute (inverse) failed";
-        return MDG_EHIP;
-    }
+    if (ctx->convOn)
+        RETCHK(mdg_conv64(ctx, ctx->gridU, nullptr, false));
+    else
+        RETCHK(fft_conv64(ctx, ctx->gridU, nullptr));
     const double f2 = 2.0 * (TWOPI / ctx->B.vol) * ctx->P.chargeConst;
     hipLaunchKernelGGL(k_hvp_gather, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, ctx->P, ctx->B,
                        n, ctx->x, ctx->y, ctx->z, ctx->q, u, sv, ctx->grid64, ctx->gridU, f2, hu,
@@ -1711,10 +1794,17 @@ k_b_spread_tiles(MdgParams Pm, const int *__restrict__ mesh, const int *__restri
         if (lane == 0) off[nbt] = run;
     }
     __syncthreads();
+    __shared__ SpreadLds<P, float> S;
     const int ncand = off[nbt], nout = binNOut[0];
     for (int c0 = 0; c0 < ncand + nout; c0 += blockDim.x) {
         const int c = c0 + threadIdx.x;
-        if (c < ncand + nout) {
+        if (threadIdx.x == 0) S.cnt = 0;
+        __syncthreads();
+        bool hit = c < ncand + nout;
+        SplineAtom<P> A = {};
+        float ql = 0.f;
+        unsigned row[3] = {0, 0, 0};
+        if (hit) {
             int l;
             if (c < ncand) {
                 int lo = 0, hi = nbt;   // off[lo] <= c < off[hi]
@@ -1727,31 +1817,21 @@ k_b_spread_tiles(MdgParams Pm, const int *__restrict__ mesh, const int *__restri
             } else {
                 l = binOut[c - ncand];
             }
-            SplineAtom<P> S;
-            spline_load<P>(splI, splB, nullptr, Pm.n, l, false, S);
+            const int4 bi = splI[l];
             // the list of atoms outside the buckets is shared by all replicas
-            if (c >= ncand && splI[l].w != r) continue;
-            const float ql = (float)q[l];
-#pragma unroll
-            for (int i = 0; i < P; i++) {
-                const int lx = wrap_index(S.base[0] - i, m) - X0;
-                if (lx < 0 || lx >= T) continue;
-                const float qa = ql * S.b[0][i];
-#pragma unroll
-                for (int j = 0; j < P; j++) {
-                    const int ly = wrap_index(S.base[1] - j, m) - Y0;
-                    if (ly < 0 || ly >= T) continue;
-                    const float qb = qa * S.b[1][j];
-#pragma unroll
-                    for (int k = 0; k < P; k++) {
-                        const int lz = wrap_index(S.base[2] - k, m) - Z0;
-                        if (lz < 0 || lz >= T) continue;
-                        const long long v = __double2ll_rn((double)(qb * S.b[2][k]) * MDG_QSCALE);
-                        atomicAdd(&acc[(lx * T + ly) * T + lz], (unsigned long long)v);
-                    }
-                }
+            hit = c < ncand || bi.w == r;
+            row[0] = spread_rows<P>(bi.x, m, X0, hit);
+            row[1] = spread_rows<P>(bi.y, m, Y0, hit);
+            row[2] = spread_rows<P>(bi.z, m, Z0, hit);
+            if (hit) {
+                ql = (float)q[l];
+                spline_load<P>(splI, splB, nullptr, Pm.n, l, false, A);
             }
         }
+        spread_put<P, float>(S, hit, ql, A.b[0], A.b[1], A.b[2], row[0], row[1], row[2]);
+        __syncthreads();
+        spread_add<P, float>(S, S.cnt, acc);
+        __syncthreads();
     }
     __syncthreads();
     const long base = gridOff[r];

@@ -1,0 +1,108 @@
+"""Kernels at the sizes where their tiles, remainders and dispatch rules change,
+against the FP64 oracle.
+
+Bars: lists are the oracle's entry for entry; FP64 energies and forces agree to
+1e-12 relative, the repository's bar for sums that differ in order only (n terms
+of one sign leave at most n eps, 3e-13 at the 1,026 atoms here; the transforms'
+log2(N) rounding steps of 1e-16 lie below that)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import mdbas_amd as M
+import oracle as O
+from mdbas_amd import configs
+from test_zz_no_alloc import Hip, relerr
+
+pytestmark = pytest.mark.gpu
+
+
+def water(nw, cut, delr, **kw):
+    L = (nw / 0.0334) ** (1 / 3)
+    return configs.build(dict(configs.COMMON, name=f"w{nw}", n_waters=nw, L=L, seed=nw,
+                              timeStep=0.002, precision="fp64", **dict(
+                                  dict(grid=20, cutOff=cut, cutOn=cut - 1.5, delr=delr,
+                                       alpha=0.35), **kw)))
+
+
+# Meshes of the in-LDS convolution (every radix, unequal edges, the largest
+# plane) and of the library transforms (odd index 3, a factor 7, a plane above
+# the limit); spline orders of the binned spreading and of the general one.
+@pytest.mark.parametrize("mesh,order", [
+    ((20, 20, 20), 4), ((24, 30, 36), 4), ((45, 27, 32), 4), ((50, 64, 18), 4), ((32, 18, 40), 6),
+    ((25, 48, 54), 8), ((80, 80, 80), 4), ((18, 20, 22), 4), ((20, 24, 25), 4), ((28, 20, 20), 4),
+    ((18, 96, 90), 4), ((24, 20, 32), 10)])
+def test_spme_meshes(mesh, order, monkeypatch):
+    wb = water(216, 7.0, 1.0, nbsp=order)
+    print("mesh", mesh, order, flush=True)
+    o = O.OracleSystem(wb)
+    o.p.m1, o.p.m2, o.p.m3 = mesh
+    made = M.reference_structs
+
+    def structs(*a):
+        s = made(*a)
+        s[3].m1max, s[3].m2max, s[3].m3max = mesh
+        return s
+
+    monkeypatch.setattr(M, "reference_structs", structs)
+    ctx = M.Context(wb)
+    # twice on moved positions: the second call finds what the first one left
+    for shift in (0.0, 0.3):
+        x, y, z = wb.x + shift, wb.y - 2 * shift, wb.z + 3 * shift
+        er, fr, st, vr = o.spme(x, y, z)
+        eg, fg, sg, vg = ctx.spme_energy(x, y, z)
+        assert eg == pytest.approx(er, rel=1e-12)
+        assert vg == pytest.approx(vr, rel=1e-10)
+        assert np.allclose(sg[[0, 3, 5]], st[[0, 3, 5]], rtol=1e-10)
+        # off the diagonal the half spectrum counts a point with one index at
+        # m/2 twice with one sign, the full one once with each; those points hold
+        # exp(-pi^2 m^2 / (4 a^2 L^2)) of the sum: 7e-9 each way for m = 18, the
+        # shortest axis here (4e-7 for 16), with L = 18.6 A and even orders (an
+        # odd order's spline transform vanishes there)
+        assert np.allclose(sg, st, rtol=1e-10, atol=1e-7 * np.abs(st).max())
+        assert relerr(fg, fr) < 1e-12
+    ctx.close()
+
+
+# 33 to 1,026 atoms: below one row group, one past 64 and 128, both sides of
+# 1,024 (the offsets' block), lists with one-entry remainders.
+@pytest.mark.parametrize("nw", [11, 21, 22, 43, 86, 341, 342])
+def test_reference_list_sizes(nw):
+    wb = water(nw, 2.6 if nw < 30 else 3.4, 0.4)
+    print("atoms", wb.n, flush=True)
+    o = O.OracleSystem(wb)
+    x, y, z = wb.x.copy(), wb.y.copy(), wb.z.copy()
+    nl, np_, no = o.build_list(x, y, z)
+    ctx = M.Context(wb)
+    gx, gy, gz = wb.x.copy(), wb.y.copy(), wb.z.copy()
+    gnl, gnp, gno, _, _ = ctx.makelist(gx, gy, gz)
+    assert np.array_equal(gnl, nl) and np.array_equal(gnp, np_) and np.array_equal(gno, no)
+    f_o, e_o = o.energy(x, y, z)
+    f_g, e_g = ctx.energy(x, y, z, nl, np_, no)
+    assert relerr(f_g, f_o) < 1e-12
+    # the device-resident path: its own list, cut into chunks by its length
+    ctx.upload(x, y, z, wb.vx, wb.vy, wb.vz)
+    e_d = ctx.initial_energy()
+    terms = sum(abs(e_o[k]) for k in ("eDir", "eRec", "eCorr", "vdw"))
+    assert e_d.nInCut == e_o["nInCut"]
+    assert abs(e_d.pot - e_o["pot"]) < 1e-12 * terms
+    for elec in (2, 3, 4):
+        f_n, e_n = o.nonbond_energy(elec, x, y, z)
+        f_g, e_g = ctx.nonbond_energy(elec, x, y, z, nl, np_, no)
+        assert relerr(f_g, f_n) < 1e-12
+    ctrl, param, pbc = ctx.ctrl, ctx.param, ctx.pbc
+    ctrl.elecType = 4
+    ctx.close()
+    # the call that allocates nothing, on the caller's device arrays
+    hip = Hip()
+    zero = np.zeros(wb.n)
+    dev = [hip.put(a) for a in (x, y, z, zero, zero, zero, wb.q, wb.eps, wb.sig, nl, np_, no)]
+    en = hip.put(np.zeros(4))
+    hip.sync()
+    assert M.load().mdg_nonbond_energy_noalloc(C.byref(ctrl), C.byref(param), C.byref(pbc), *dev,
+                                               en, None) == 0
+    hip.sync()
+    f = np.stack([hip.get(p, zero) for p in dev[3:6]])
+    hip.free()
+    assert relerr(f, f_n) < 1e-12
