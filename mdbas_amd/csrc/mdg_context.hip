@@ -258,6 +258,7 @@ int mdg_build_exclusions(mdg_ctx *ctx, int nBond, const MDG_BOND *bond, int nCon
 int mdg_upload_exclusions(mdg_ctx *ctx)
 {
     const int ne = (int)ctx->hExLst.size();
+    ctx->exReady = false;
     if (ne > ctx->nExcl || !ctx->exLst) {
         if (ctx->exLst) HIPCHK(hipFree(ctx->exLst));
         RETCHK(dmalloc(ctx, &ctx->exLst, ne + 1));
@@ -300,20 +301,26 @@ int mdg_upload_exclusions(mdg_ctx *ctx)
     if (!ctx->exSymOff) RETCHK(dmalloc(ctx, &ctx->exSymOff, n + 1));
     RETCHK(h2d(ctx, ctx->exSymOff, off.data(), n + 1));
     RETCHK(h2d(ctx, ctx->exSymLst, lst.data(), off[n]));
-    return sync(ctx);
+    RETCHK(sync(ctx));
+    ctx->exReady = true;
+    return MDG_OK;
 }
 
-// Exclusion table from the reference's (exclList, exclPair) arguments.
+// Exclusion table from the reference's (exclList, exclPair) arguments; a table
+// equal to the one on the device, entry for entry, is not laid out again.
 static int exclusions_from_args(mdg_ctx *ctx, int **exclList, const int *exclPair)
 {
     const int n = ctx->n;
-    ctx->hExOff.assign(n + 1, 0);
-    ctx->hExLst.clear();
+    std::vector<int> off(n + 1, 0), lst;
+    lst.reserve(ctx->hExLst.size());
     for (int i = 0; i < n; i++) {
-        ctx->hExOff[i] = (int)ctx->hExLst.size();
-        for (int k = 0; k < exclPair[i]; k++) ctx->hExLst.push_back(exclList[i][k]);
+        off[i] = (int)lst.size();
+        if (exclPair[i] > 0) lst.insert(lst.end(), exclList[i], exclList[i] + exclPair[i]);
     }
-    ctx->hExOff[n] = (int)ctx->hExLst.size();
+    off[n] = (int)lst.size();
+    if (ctx->exReady && off == ctx->hExOff && lst == ctx->hExLst) return MDG_OK;
+    ctx->hExOff.swap(off);
+    ctx->hExLst.swap(lst);
     return mdg_upload_exclusions(ctx);
 }
 
@@ -525,6 +532,7 @@ extern "C" void mdg_destroy(mdg_ctx *ctx)
         if (ctx->graphExec[k]) hipGraphExecDestroy(ctx->graphExec[k]);
     mdg_spme_free(ctx);
     mdg_bonded_free(ctx);
+    mdg_xfer_free(ctx);
     void *ptrs[] = {ctx->x, ctx->y, ctx->z, ctx->vx, ctx->vy, ctx->vz, ctx->fx, ctx->fy, ctx->fz,
                     ctx->q, ctx->eps, ctx->sig, ctx->mass, ctx->rmass, ctx->frozen, ctx->nAtConst,
                     ctx->ca, ctx->cb, ctx->rc2, ctx->dd, ctx->grpAtomOff, ctx->grpAtoms,
@@ -807,6 +815,27 @@ extern "C" int mdg_set_nonbond_params(mdg_ctx *ctx, const double q[], const doub
     return sync(ctx);
 }
 
+static void put_xyzq(mdg_ctx *ctx, MdgXfer &X, const double *x, const double *y, const double *z,
+                     const double *q, const double *eps, const double *sig)
+{
+    const int n = ctx->n;
+    X.put(ctx->x, x, n);
+    X.put(ctx->y, y, n);
+    X.put(ctx->z, z, n);
+    if (q) X.put(ctx->q, q, n);
+    if (eps) X.put(ctx->eps, eps, n);
+    if (sig) X.put(ctx->sig, sig, n);
+}
+
+// Forces to or from the device (null on the way up: zeros).
+static void put_forces(mdg_ctx *ctx, MdgXfer &X, const double *fx, const double *fy,
+                       const double *fz)
+{
+    X.put(ctx->fx, fx, ctx->n);
+    X.put(ctx->fy, fy, ctx->n);
+    X.put(ctx->fz, fz, ctx->n);
+}
+
 // ---------------------------------------------------------------- drop-in: makelist
 
 static int download_ref_list(mdg_ctx *ctx, MDG_NEIGH *neigh, int **neighList, int **neighPair,
@@ -827,9 +856,11 @@ static int download_ref_list(mdg_ctx *ctx, MDG_NEIGH *neigh, int **neighList, in
     }
     if (!*neighList || !*neighPair || !*neighOrder) return MDG_EARG;
     RETCHK(d2h(ctx, *neighList, R.neighList, R.count));
-    RETCHK(d2h(ctx, *neighPair, R.neighPair, n));
-    RETCHK(d2h(ctx, *neighOrder, R.neighOrder, n));
-    return sync(ctx);
+    MdgXfer D(false);
+    D.put(R.neighPair, *neighPair, n);
+    D.put(R.neighOrder, *neighOrder, n);
+    RETCHK(D.fetch(ctx, 0));
+    return D.deliver(ctx);
 }
 
 extern "C" int mdg_makelist(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, MDG_PBC *box,
@@ -873,9 +904,9 @@ extern "C" int mdg_makelist(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, MDG_
             *neighList14 = (int *)malloc(std::max<size_t>(l14.size(), 1) * sizeof(int));
             std::copy(l14.begin(), l14.end(), *neighList14);
         }
-        RETCHK(h2d(ctx, ctx->x, (const double *)x, n));
-        RETCHK(h2d(ctx, ctx->y, (const double *)y, n));
-        RETCHK(h2d(ctx, ctx->z, (const double *)z, n));
+        MdgXfer X(true);
+        put_xyzq(ctx, X, x, y, z, nullptr, nullptr, nullptr);
+        RETCHK(X.up(ctx));
         RETCHK(mdg_build_ref_list(ctx, true));
         if (ctx->keyLink) {
             // list.c:1927: the first link-cell build wraps the coordinates
@@ -887,9 +918,9 @@ extern "C" int mdg_makelist(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, MDG_
         RETCHK(download_ref_list(ctx, neigh, neighList, neighPair, neighOrder, true));
         ctrl->newjob = 0;
     } else if (param->step % neigh->update == 0) {
-        RETCHK(h2d(ctx, ctx->x, (const double *)x, n));
-        RETCHK(h2d(ctx, ctx->y, (const double *)y, n));
-        RETCHK(h2d(ctx, ctx->z, (const double *)z, n));
+        MdgXfer X(true);
+        put_xyzq(ctx, X, x, y, z, nullptr, nullptr, nullptr);
+        RETCHK(X.up(ctx));
         RETCHK(mdg_build_ref_list(ctx, false));
         RETCHK(download_ref_list(ctx, neigh, neighList, neighPair, neighOrder, false));
     }
@@ -905,13 +936,14 @@ extern "C" int mdg_makelist(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, MDG_
 
 // ---------------------------------------------------------------- drop-in: energies
 
-// Upload the list in the reference format with per-position offsets.
-static int upload_ref_list(mdg_ctx *ctx, const int *neighList, const int *neighPair,
-                           const int *neighOrder)
+// The list in the reference format with per-position offsets (off, the caller's
+// until X has gone up): the list itself at once, the rest with X.
+static int upload_ref_list(mdg_ctx *ctx, MdgXfer &X, std::vector<long> &off, const int *neighList,
+                           const int *neighPair, const int *neighOrder)
 {
     const int n = ctx->n;
     RefList &R = ctx->rl;
-    std::vector<long> off(n + 1, 0);
+    off.assign(n + 1, 0);
     for (int l = 0; l < n; l++) off[l + 1] = off[l] + neighPair[neighOrder[l]];
     const long total = off[n];
     if (!R.off) RETCHK(dmalloc(ctx, &R.off, n + 1));
@@ -924,23 +956,9 @@ static int upload_ref_list(mdg_ctx *ctx, const int *neighList, const int *neighP
         RETCHK(dmalloc(ctx, &R.neighList, R.cap));
     }
     R.count = total;
-    RETCHK(h2d(ctx, R.off, off.data(), n + 1));
-    RETCHK(h2d(ctx, R.neighOrder, neighOrder, n));
-    RETCHK(h2d(ctx, R.neighList, neighList, total));
-    return sync(ctx);
-}
-
-static int upload_xyzq(mdg_ctx *ctx, const double *x, const double *y, const double *z,
-                       const double *q, const double *eps, const double *sig)
-{
-    const int n = ctx->n;
-    RETCHK(h2d(ctx, ctx->x, x, n));
-    RETCHK(h2d(ctx, ctx->y, y, n));
-    RETCHK(h2d(ctx, ctx->z, z, n));
-    if (q) RETCHK(h2d(ctx, ctx->q, q, n));
-    if (eps) RETCHK(h2d(ctx, ctx->eps, eps, n));
-    if (sig) RETCHK(h2d(ctx, ctx->sig, sig, n));
-    return MDG_OK;
+    X.put(R.off, off.data(), n + 1);
+    X.put(R.neighOrder, neighOrder, n);
+    return h2d(ctx, R.neighList, neighList, total);
 }
 
 static int refresh_charge_terms(mdg_ctx *ctx, const double *q)
@@ -956,18 +974,18 @@ extern "C" int mdg_spme_energy(mdg_ctx *ctx, MDG_PARAM *param, MDG_EWALD *ewald,
 {
     (void)param; (void)ewald; (void)box;
     if (!ctx || !x || !fx || !q || !ctx->theta) return MDG_EARG;
-    const int n = ctx->n;
-    RETCHK(upload_xyzq(ctx, x, y, z, q, nullptr, nullptr));
+    MdgXfer X(true), D(false);
+    put_xyzq(ctx, X, x, y, z, q, nullptr, nullptr);
+    put_forces(ctx, X, fx, fy, fz);
+    RETCHK(X.up(ctx));
     RETCHK(refresh_charge_terms(ctx, q));
-    RETCHK(h2d(ctx, ctx->fx, (const double *)fx, n));
-    RETCHK(h2d(ctx, ctx->fy, (const double *)fy, n));
-    RETCHK(h2d(ctx, ctx->fz, (const double *)fz, n));
-    double e[8];
-    RETCHK(mdg_spme64(ctx, ctx->fx, ctx->fy, ctx->fz, e));
-    RETCHK(d2h(ctx, fx, ctx->fx, n));
-    RETCHK(d2h(ctx, fy, ctx->fy, n));
-    RETCHK(d2h(ctx, fz, ctx->fz, n));
-    RETCHK(sync(ctx));
+    RETCHK(mdg_spme64(ctx, ctx->fx, ctx->fy, ctx->fz));
+    double e[8], h[S_COUNT];
+    D.put(ctx->scal, h, S_COUNT);
+    put_forces(ctx, D, fx, fy, fz);
+    RETCHK(D.fetch(ctx, 1));
+    RETCHK(D.deliver(ctx));
+    mdg_spme64_sums(ctx, h + S_EREC, e);
     if (eEwaldRec) *eEwaldRec = e[0];
     if (virEwaldRec) *virEwaldRec = e[1];
     if (stress)
@@ -978,43 +996,46 @@ extern "C" int mdg_spme_energy(mdg_ctx *ctx, MDG_PARAM *param, MDG_EWALD *ewald,
 // energy.c:450-643 on the device: uploads positions, parameters, list and
 // exclusions and forces fx (the caller's +=), runs SPME (keyEwald 2), the
 // real-space pairs and the excluded-pair correction into ctx->fx..; the
-// forces stay on the device.  e[0..3] = elec, vdw, virelec, virvdw to add.
+// forces and the sums (scal) stay on the device.  fx null: from zero.
 static int ewald_on_device(mdg_ctx *ctx, const MDG_CTRL *ctrl, const double *x, const double *y,
                            const double *z, const double *fx, const double *fy, const double *fz,
                            const double *q, const double *eps, const double *sig,
                            const int *neighList, const int *neighPair, const int *neighOrder,
-                           int **exclList, const int *exclPair, double e[4])
+                           int **exclList, const int *exclPair)
 {
-    const int n = ctx->n;
     if (ctrl->keyEwald == 1) {
         ctx->err = "classic k-space Ewald (keyEwald 1) is not on this path";
         return MDG_EUNSUPPORTED;
     }
     ctx->P.vdwOn = ctrl->vdwType == 2;
-    RETCHK(upload_xyzq(ctx, x, y, z, q, eps, sig));
-    RETCHK(upload_ref_list(ctx, neighList, neighPair, neighOrder));
+    MdgXfer X(true);
+    std::vector<long> off;
+    put_xyzq(ctx, X, x, y, z, q, eps, sig);
+    put_forces(ctx, X, fx, fy, fz);
+    RETCHK(upload_ref_list(ctx, X, off, neighList, neighPair, neighOrder));
     RETCHK(exclusions_from_args(ctx, exclList, exclPair));
-    RETCHK(h2d(ctx, ctx->fx, fx, n));
-    RETCHK(h2d(ctx, ctx->fy, fy, n));
-    RETCHK(h2d(ctx, ctx->fz, fz, n));
-    double erec[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    RETCHK(X.up(ctx));
     if (ctrl->keyEwald == 2) {
         if (!ctx->theta) return MDG_EARG;
         RETCHK(refresh_charge_terms(ctx, q));
-        RETCHK(mdg_spme64(ctx, ctx->fx, ctx->fy, ctx->fz, erec));
+        RETCHK(mdg_spme64(ctx, ctx->fx, ctx->fy, ctx->fz));
     }
     RETCHK(mdg_pair_ref64(ctx, 0, ctx->fx, ctx->fy, ctx->fz, ctx->rl.neighList, ctx->rl.off,
                           ctx->rl.neighOrder, ctx->scal + S_REF));
-    RETCHK(mdg_excl_corr64(ctx, ctx->fx, ctx->fy, ctx->fz, ctx->scal + S_REFCORR));
-    double s[8];
-    RETCHK(d2h(ctx, s, ctx->scal + S_REF, 8));
-    RETCHK(sync(ctx));
+    return mdg_excl_corr64(ctx, ctx->fx, ctx->fy, ctx->fz, ctx->scal + S_REFCORR);
+}
+
+// e[0..3] = elec, vdw, virelec, virvdw to add, from a host copy of scal.
+static void ewald_sums(const mdg_ctx *ctx, const MDG_CTRL *ctrl, const double *h, double e[4])
+{
+    const double *s = h + S_REF;
+    double erec[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    if (ctrl->keyEwald == 2) mdg_spme64_sums(ctx, h + S_EREC, erec);
     // energy.c:623-627
     e[0] = s[0] + erec[0] + s[6];
     e[1] = s[1];
     e[2] = s[2] + erec[1] + s[7];
     e[3] = s[3];
-    return MDG_OK;
 }
 
 // energy.c:216-345 on the device (see ewald_on_device).
@@ -1022,37 +1043,21 @@ static int nonbond_on_device(mdg_ctx *ctx, const MDG_CTRL *ctrl, const double *x
                              const double *z, const double *fx, const double *fy,
                              const double *fz, const double *q, const double *eps,
                              const double *sig, const int *neighList, const int *neighPair,
-                             const int *neighOrder, double e[4])
+                             const int *neighOrder)
 {
-    const int n = ctx->n;
     // energy.c:45-65: FULL and NOELEC evaluate no electrostatics
     int et = ctrl->elecType;
     if (et == 0) et = 1;
     if (et < 1 || et > 4) return MDG_EUNSUPPORTED;
     ctx->P.vdwOn = ctrl->vdwType == 2;
-    RETCHK(upload_xyzq(ctx, x, y, z, q, eps, sig));
-    RETCHK(upload_ref_list(ctx, neighList, neighPair, neighOrder));
-    RETCHK(h2d(ctx, ctx->fx, fx, n));
-    RETCHK(h2d(ctx, ctx->fy, fy, n));
-    RETCHK(h2d(ctx, ctx->fz, fz, n));
-    RETCHK(mdg_pair_ref64(ctx, et, ctx->fx, ctx->fy, ctx->fz, ctx->rl.neighList, ctx->rl.off,
-                          ctx->rl.neighOrder, ctx->scal + S_REF));
-    double s[6];
-    RETCHK(d2h(ctx, s, ctx->scal + S_REF, 6));
-    RETCHK(sync(ctx));
-    e[0] = s[0];
-    e[1] = s[1];
-    e[2] = s[2];
-    e[3] = s[3];
-    return MDG_OK;
-}
-
-static int download_forces(mdg_ctx *ctx, double *fx, double *fy, double *fz)
-{
-    RETCHK(d2h(ctx, fx, ctx->fx, ctx->n));
-    RETCHK(d2h(ctx, fy, ctx->fy, ctx->n));
-    RETCHK(d2h(ctx, fz, ctx->fz, ctx->n));
-    return sync(ctx);
+    MdgXfer X(true);
+    std::vector<long> off;
+    put_xyzq(ctx, X, x, y, z, q, eps, sig);
+    put_forces(ctx, X, fx, fy, fz);
+    RETCHK(upload_ref_list(ctx, X, off, neighList, neighPair, neighOrder));
+    RETCHK(X.up(ctx));
+    return mdg_pair_ref64(ctx, et, ctx->fx, ctx->fy, ctx->fz, ctx->rl.neighList, ctx->rl.off,
+                          ctx->rl.neighOrder, ctx->scal + S_REF);
 }
 
 extern "C" int mdg_ewald_energy(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, MDG_ENERGY *ener,
@@ -1065,10 +1070,15 @@ extern "C" int mdg_ewald_energy(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, 
     (void)param; (void)ewald;
     if (!ctx || !ctrl || !ener || !x || !fx || !q || !neighPair || !neighOrder) return MDG_EARG;
     if (box) RETCHK(mdg_refresh_box(ctx, box));
-    double e[4];
     RETCHK(ewald_on_device(ctx, ctrl, x, y, z, fx, fy, fz, q, eps, sig, neighList, neighPair,
-                           neighOrder, exclList, exclPair, e));
-    RETCHK(download_forces(ctx, fx, fy, fz));
+                           neighOrder, exclList, exclPair));
+    double e[4], h[S_COUNT];
+    MdgXfer D(false);
+    D.put(ctx->scal, h, S_COUNT);
+    put_forces(ctx, D, fx, fy, fz);
+    RETCHK(D.fetch(ctx, 1));
+    RETCHK(D.deliver(ctx));
+    ewald_sums(ctx, ctrl, h, e);
     ener->elec += e[0];
     ener->vdw += e[1];
     ener->virelec += e[2];
@@ -1086,10 +1096,15 @@ extern "C" int mdg_nonbond_energy(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param
     (void)param;
     if (!ctx || !ctrl || !ener || !x || !fx || !q || !neighPair || !neighOrder) return MDG_EARG;
     if (box) RETCHK(mdg_refresh_box(ctx, box));
-    double e[4];
     RETCHK(nonbond_on_device(ctx, ctrl, x, y, z, fx, fy, fz, q, eps, sig, neighList, neighPair,
-                             neighOrder, e));
-    RETCHK(download_forces(ctx, fx, fy, fz));
+                             neighOrder));
+    double h[S_COUNT];
+    MdgXfer D(false);
+    D.put(ctx->scal, h, S_COUNT);
+    put_forces(ctx, D, fx, fy, fz);
+    RETCHK(D.fetch(ctx, 1));
+    RETCHK(D.deliver(ctx));
+    const double *e = h + S_REF;
     ener->elec += e[0];
     ener->vdw += e[1];
     ener->virelec += e[2];
@@ -1123,20 +1138,14 @@ extern "C" int mdg_energy(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, MDG_EN
     box->stress1 = box->stress2 = box->stress3 = box->stress4 = box->stress5 = 0.;
     box->stress6 = box->stress7 = box->stress8 = box->stress9 = 0.;
     const int n = ctx->n;
-    std::vector<double> zero(n, 0.);
-    // energy.c:151-165: Ewald or plain nonbonded terms (into the zeroed
+    // energy.c:151-165: Ewald or plain nonbonded terms (into zeroed
     // forces), each followed by its 1-4 pairs when keyNb14 is set
-    double e[4];
     if (ctrl->keyEwald != 0)
-        RETCHK(ewald_on_device(ctx, ctrl, x, y, z, zero.data(), zero.data(), zero.data(), q, eps,
-                               sig, neighList, neighPair, neighOrder, exclList, exclPair, e));
+        RETCHK(ewald_on_device(ctx, ctrl, x, y, z, nullptr, nullptr, nullptr, q, eps, sig,
+                               neighList, neighPair, neighOrder, exclList, exclPair));
     else
-        RETCHK(nonbond_on_device(ctx, ctrl, x, y, z, zero.data(), zero.data(), zero.data(), q,
-                                 eps, sig, neighList, neighPair, neighOrder, e));
-    ener->elec += e[0];
-    ener->vdw += e[1];
-    ener->virelec += e[2];
-    ener->virvdw += e[3];
+        RETCHK(nonbond_on_device(ctx, ctrl, x, y, z, nullptr, nullptr, nullptr, q, eps, sig,
+                                 neighList, neighPair, neighOrder));
     // energy.c:157-189: 1-4 pairs, bonds, angles, Urey-Bradley, dihedrals,
     // impropers, all in one device kernel
     MdgBonded &D = ctx->bd;
@@ -1148,9 +1157,20 @@ extern "C" int mdg_energy(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, MDG_EN
                              param->nDihedral, dihe, param->nImproper, impr, n14, neighList14,
                              eps14, sig14));
     RETCHK(mdg_bonded_forces(ctx, ctx->fx, ctx->fy, ctx->fz, nullptr));
-    double b[11];
-    RETCHK(d2h(ctx, b, ctx->scal + S_BONDED, 11));
-    RETCHK(download_forces(ctx, fx, fy, fz));
+    // one transfer and one wait for the forces and every sum
+    double e[4], h[S_COUNT];
+    const double *b = h + S_BONDED;
+    MdgXfer Y(false);
+    Y.put(ctx->scal, h, S_COUNT);
+    put_forces(ctx, Y, fx, fy, fz);
+    RETCHK(Y.fetch(ctx, 1));
+    RETCHK(Y.deliver(ctx));
+    if (ctrl->keyEwald != 0) ewald_sums(ctx, ctrl, h, e);
+    else std::copy(h + S_REF, h + S_REF + 4, e);
+    ener->elec += e[0];
+    ener->vdw += e[1];
+    ener->virelec += e[2];
+    ener->virvdw += e[3];
     ener->elec += b[7];
     ener->vdw += b[8];
     ener->virelec += b[9];
@@ -1196,37 +1216,35 @@ extern "C" int mdg_vv_integrate(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, 
                                 std::vector<double>(n, 0.).data(), mass, rmass, nullptr, nAtConst,
                                 constList, param->nConst));
     }
-    RETCHK(h2d(ctx, ctx->mass, (const double *)mass, n));
-    RETCHK(h2d(ctx, ctx->rmass, (const double *)rmass, n));
-    if (nAtConst) RETCHK(h2d(ctx, ctx->nAtConst, (const int *)nAtConst, n));
-    RETCHK(upload_xyzq(ctx, x, y, z, nullptr, nullptr, nullptr));
-    RETCHK(h2d(ctx, ctx->vx, (const double *)vx, n));
-    RETCHK(h2d(ctx, ctx->vy, (const double *)vy, n));
-    RETCHK(h2d(ctx, ctx->vz, (const double *)vz, n));
-    RETCHK(h2d(ctx, ctx->fx, (const double *)fx, n));
-    RETCHK(h2d(ctx, ctx->fy, (const double *)fy, n));
-    RETCHK(h2d(ctx, ctx->fz, (const double *)fz, n));
+    MdgXfer X(true), D(false);
+    X.put(ctx->mass, mass, n);
+    X.put(ctx->rmass, rmass, n);
+    if (nAtConst) X.put(ctx->nAtConst, nAtConst, n);
+    put_xyzq(ctx, X, x, y, z, nullptr, nullptr, nullptr);
+    X.put(ctx->vx, vx, n);
+    X.put(ctx->vy, vy, n);
+    X.put(ctx->vz, vz, n);
+    put_forces(ctx, X, fx, fy, fz);
+    RETCHK(X.up(ctx));
+    int c[CTRL_WORDS];
+    double h[S_COUNT];
+    D.put(ctx->ctrl, c, CTRL_WORDS);
+    D.put(ctx->scal, h, S_COUNT);
+    put_xyzq(ctx, D, x, y, z, nullptr, nullptr, nullptr);
+    D.put(ctx->vx, vx, n);
+    D.put(ctx->vy, vy, n);
+    D.put(ctx->vz, vz, n);
     double kin[8] = {0}, vs = 0.;
     if (ens != 0) {
         // integrate.c:1495-1506: the thermostat and barostat integrators
         RETCHK(mdg_vv_ensemble(ctx, param, ener, box, bath, ens, stage));
-        RETCHK(d2h(ctx, x, ctx->x, n));
-        RETCHK(d2h(ctx, y, ctx->y, n));
-        RETCHK(d2h(ctx, z, ctx->z, n));
-        RETCHK(d2h(ctx, vx, ctx->vx, n));
-        RETCHK(d2h(ctx, vy, ctx->vy, n));
-        RETCHK(d2h(ctx, vz, ctx->vz, n));
-        return sync(ctx);
+        RETCHK(D.fetch(ctx, 2));
+        return D.deliver(ctx);
     }
-    int st = mdg_vv_stage(ctx, stage, ctx->fx, ctx->fy, ctx->fz, kin, &vs, true);
-    if (st) return st;
-    RETCHK(d2h(ctx, x, ctx->x, n));
-    RETCHK(d2h(ctx, y, ctx->y, n));
-    RETCHK(d2h(ctx, z, ctx->z, n));
-    RETCHK(d2h(ctx, vx, ctx->vx, n));
-    RETCHK(d2h(ctx, vy, ctx->vy, n));
-    RETCHK(d2h(ctx, vz, ctx->vz, n));
-    RETCHK(sync(ctx));
+    RETCHK(mdg_vv_stage(ctx, stage, ctx->fx, ctx->fy, ctx->fz, nullptr, nullptr, true));
+    RETCHK(D.fetch(ctx, 2));
+    RETCHK(mdg_vv_result(ctx, c, h, kin, &vs));
+    RETCHK(D.deliver(ctx));
     if (stage == 1) {
         if (param->nConst > 0) ener->virshake = vs;
     } else {

@@ -617,7 +617,8 @@ int mdg_vir_rows(const mdg_ctx *ctx)
 // Runs one VV stage on the device state with forces fx.. (device, atom
 // order).  Per-group SHAKE virials go to grpVir (stage 1) and per-block
 // kinetic partials to epart + PART_KIN (stage 2); with sync the sums land
-// in scal[S_VIRSHAKE] and scal[S_KIN..S_KIN+6] and are returned.
+// in scal[S_VIRSHAKE] and scal[S_KIN..S_KIN+6] and, unless both outputs are
+// null (the caller fetches ctrl and scal for mdg_vv_result), are returned.
 int mdg_vv_stage(mdg_ctx *ctx, int stage, double *fx, double *fy, double *fz, double *kin_out,
                  double *virshake_out, bool sync, const FinArgs *fin, const VvOpts *opt)
 {
@@ -807,29 +808,35 @@ int mdg_vv_stage(mdg_ctx *ctx, int stage, double *fx, double *fy, double *fz, do
         LAUNCHCHK();
         if (sync) RETCHK(mdg_reduce_partials(ctx, A.part, nb, 7, ctx->scal + S_KIN));
     }
-    if (sync) {
+    if (sync && (kin_out || virshake_out)) {
         int c[CTRL_WORDS];
-        double s[8];
-        HIPCHK(hipMemcpyAsync(c, ctx->ctrl, sizeof c, hipMemcpyDeviceToHost, ctx->stream));
-        HIPCHK(hipMemcpyAsync(s, ctx->scal + S_KIN, 8 * sizeof(double), hipMemcpyDeviceToHost,
-                              ctx->stream));
-        double vs = 0.;
-        HIPCHK(hipMemcpyAsync(&vs, ctx->scal + S_VIRSHAKE, sizeof(double), hipMemcpyDeviceToHost,
-                              ctx->stream));
-        HIPCHK(hipStreamSynchronize(ctx->stream));
-        if (kin_out) {
-            for (int k = 0; k < 7; k++) kin_out[k] = s[k];
-            kin_out[0] *= 0.5;
-        }
-        if (virshake_out) *virshake_out = vs;
-        if (c[CTRL_SHAKE_FAIL]) {
-            ctx->err = "SHAKE did not converge within maxCycle";
-            return 311;
-        }
-        if (c[CTRL_SHAKE_ORDER]) {
-            ctx->err = "a constraint group re-diverged after converging";
-            return MDG_ESHAKE_ORDER;
-        }
+        double h[S_COUNT];
+        MdgXfer X(false);
+        X.put(ctx->ctrl, c, CTRL_WORDS);
+        X.put(ctx->scal, h, S_COUNT);
+        RETCHK(X.fetch(ctx, 2));
+        return mdg_vv_result(ctx, c, h, kin_out, virshake_out);
+    }
+    return MDG_OK;
+}
+
+// A synchronous stage's sums from host copies of ctrl and scal: the kinetic
+// energy and stress, the SHAKE virial, or the SHAKE error.
+int mdg_vv_result(mdg_ctx *ctx, const int *c, const double *scal, double *kin_out,
+                  double *virshake_out)
+{
+    if (kin_out) {
+        for (int k = 0; k < 7; k++) kin_out[k] = scal[S_KIN + k];
+        kin_out[0] *= 0.5;
+    }
+    if (virshake_out) *virshake_out = scal[S_VIRSHAKE];
+    if (c[CTRL_SHAKE_FAIL]) {
+        ctx->err = "SHAKE did not converge within maxCycle";
+        return 311;
+    }
+    if (c[CTRL_SHAKE_ORDER]) {
+        ctx->err = "a constraint group re-diverged after converging";
+        return MDG_ESHAKE_ORDER;
     }
     return MDG_OK;
 }

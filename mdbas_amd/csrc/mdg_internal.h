@@ -202,6 +202,39 @@ struct ConvPlan {
     unsigned mMh = 0, mNz = 0, mCols = 0;
 };
 
+// Arrays of a drop-in call to or from the device (mdg_xfer.hip).
+#define MDG_XFER_SEGS 20
+struct MdgXferSeg {
+    void *dev;
+    unsigned off, bytes;
+};
+struct MdgXferTab {
+    MdgXferSeg s[MDG_XFER_SEGS];
+};
+struct MdgXfer {
+    explicit MdgXfer(bool toDevice) : in(toDevice) {}
+    void add(void *dev, void *host, size_t bytes);
+    template <typename T> void put(T *dev, const T *host, size_t cnt)
+    {
+        add(dev, const_cast<T *>(host), cnt * sizeof(T));
+    }
+    int up(struct mdg_ctx *ctx);
+    int fetch(struct mdg_ctx *ctx, int nfirst);
+    int deliver(struct mdg_ctx *ctx);
+
+  private:
+    int prepare(struct mdg_ctx *ctx);
+    int launch(struct mdg_ctx *ctx);
+    struct {
+        void *dev, *host;
+        size_t bytes, off;
+    } seg[MDG_XFER_SEGS];
+    int n = 0, first = 0;
+    size_t total = 0;
+    bool in, full = false, packed = false;
+    char *buf = nullptr;
+};
+
 struct mdg_ctx {
     int precision = MDG_FP64;
     int n = 0;
@@ -295,6 +328,9 @@ struct mdg_ctx {
     double *relPart = nullptr;
     int pairPath = 0;
     double pruneSkin = 0.;       // > 0: the mixed pair kernel may use the pruned list
+    char *xferUp = nullptr, *xferDown = nullptr;   // pinned (mdg_xfer.hip)
+    bool xferBusy = false;       // a transfer may still be reading xferUp
+    bool exReady = false;        // the device exclusion tables are hExOff / hExLst
     bool pruneSet = false;       // mdg_set_prune was called: the tuner adds no pruning of its own
     bool pruneFresh = true;      // the list was rebuilt since the last slot update
     // device steps without a rebuild (one box of three-site molecules,
@@ -644,11 +680,13 @@ double mdg_prune_candidate(const mdg_ctx *ctx);   // mdg_context.hip: the skin t
 // spme (mdg_spme.hip)
 int mdg_spme_setup(mdg_ctx *ctx);
 int mdg_spme_free(mdg_ctx *ctx);
-int mdg_spme64(mdg_ctx *ctx, double *fx, double *fy, double *fz, double eout[8]);
+int mdg_spme64(mdg_ctx *ctx, double *fx, double *fy, double *fz);
+void mdg_spme64_sums(const mdg_ctx *ctx, const double s[7], double eout[8]);
 int mdg_spme_device(mdg_ctx *ctx);   // device-resident: frx.. per atom, partials in epart
 int mdg_spme_fork(mdg_ctx *ctx);   // marks the point stream2's work starts from
 int mdg_spme_on(mdg_ctx *ctx, int (*fn)(mdg_ctx *));   // runs fn's launches on stream2 from it
 // blocks (= partial rows) of the SPME influence kernel over H half-spectrum points
+void mdg_xfer_free(mdg_ctx *ctx);      // mdg_xfer.hip
 int mdg_conv64_setup(mdg_ctx *ctx);   // mdg_conv64.hip
 int mdg_conv64_rows(const mdg_ctx *ctx);
 int mdg_conv64(mdg_ctx *ctx, double *grid, double *part, bool clearBins);
@@ -687,6 +725,8 @@ struct VvOpts {
 int mdg_vv_stage(mdg_ctx *ctx, int stage, double *fx, double *fy, double *fz, double *kin_out,
                  double *virshake_out, bool sync, const FinArgs *fin = nullptr,
                  const VvOpts *opt = nullptr);
+int mdg_vv_result(mdg_ctx *ctx, const int *ctrl, const double *scal, double *kin_out,
+                  double *virshake_out);
 // the device-resident thermostat of one step, before stage 1 (stage 1) or
 // after stage 2 (stage 2) (mdg_ensemble.hip)
 int mdg_thermo_stage(mdg_ctx *ctx, int stage);

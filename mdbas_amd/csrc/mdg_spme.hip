@@ -1328,7 +1328,9 @@ __global__ void k_sub_mean(int n, double *fx, double *fy, double *fz, const doub
     fz[i] -= sums[2] / (double)n;
 }
 
-int mdg_spme64(mdg_ctx *ctx, double *fx, double *fy, double *fz, double eout[8])
+// The FP64 reciprocal term of the drop-in calls: forces added to fx.., sums
+// left in scal + S_EREC for mdg_spme64_sums.
+int mdg_spme64(mdg_ctx *ctx, double *fx, double *fy, double *fz)
 {
     const int n = ctx->n;
     RETCHK(spme_run(ctx, false, ctx->epart + PART_INFL, ctx->epart + PART_GATHER, ctx->frx64,
@@ -1342,10 +1344,12 @@ int mdg_spme64(mdg_ctx *ctx, double *fx, double *fy, double *fz, double eout[8])
     hipLaunchKernelGGL(k_sub_mean, dim3(nblk(n, 256)), dim3(256), 0, ctx->stream, n, fx, fy, fz,
                        ctx->scal + S_FRX);
     LAUNCHCHK();
-    double s[7];
-    HIPCHK(hipMemcpyAsync(s, ctx->scal + S_EREC, 7 * sizeof(double), hipMemcpyDeviceToHost,
-                          ctx->stream));
-    HIPCHK(hipStreamSynchronize(ctx->stream));
+    return MDG_OK;
+}
+
+// Energy, virial and stress from a host copy of scal + S_EREC.
+void mdg_spme64_sums(const mdg_ctx *ctx, const double s[7], double eout[8])
+{
     // spme.c:674-697
     const double fact = (TWOPI / ctx->B.vol) * ctx->P.chargeConst;
     const double eRec = s[0];
@@ -1359,7 +1363,6 @@ int mdg_spme64(mdg_ctx *ctx, double *fx, double *fy, double *fz, double eout[8])
     eout[0] = fact * eRec + ctx->eSelf + ctx->eNet;
     eout[1] = -(st[0] + st[3] + st[5]);
     for (int k = 0; k < 6; k++) eout[2 + k] = st[k];
-    return MDG_OK;
 }
 
 // dE_rec/dq per atom (FP64, self and net-charge terms not included) into

@@ -106,3 +106,31 @@ def test_reference_list_sizes(nw):
     f = np.stack([hip.get(p, zero) for p in dev[3:6]])
     hip.free()
     assert relerr(f, f_n) < 1e-12
+
+
+# Drop-in transfers on both sides of the pinned buffer's limit (1 MiB): an
+# integrator stage crosses it between 3,790 and 3,810 molecules (92 bytes an
+# atom), the plain energies between 4,150 and 4,170 (84 bytes).
+@pytest.mark.parametrize("nw", [3790, 3810, 4150, 4170])
+def test_dropin_transfer_sizes(nw):
+    wb = water(nw, 4.0, 0.5)
+    print("atoms", wb.n, flush=True)
+    o = O.OracleSystem(wb)
+    x, y, z = wb.x.copy(), wb.y.copy(), wb.z.copy()
+    nl, np_, no = o.build_list(x, y, z)
+    ctx = M.Context(wb)
+    gx, gy, gz = wb.x.copy(), wb.y.copy(), wb.z.copy()
+    gnl, gnp, gno, _, _ = ctx.makelist(gx, gy, gz)
+    assert np.array_equal(gx, x) and np.array_equal(gnl, nl)
+    assert np.array_equal(gnp, np_) and np.array_equal(gno, no)
+    f_o, e_o = o.nonbond_energy(4, x, y, z)
+    f_g, e_g = ctx.nonbond_energy(4, x, y, z, nl, np_, no)
+    assert relerr(f_g, f_o) < 1e-12 and e_g.vdw == pytest.approx(e_o["vdw"], rel=1e-11)
+    s_o = [x, y, z, wb.vx.copy(), wb.vy.copy(), wb.vz.copy()]
+    s_g = [a.copy() for a in s_o]
+    for stage in (1, 2):
+        err, *_ = o.vv(stage, *s_o, f_o)
+        assert err == 0
+        ctx.vv_integrate(stage, *s_g, f_o.copy())
+        assert max(np.abs(a - b).max() for a, b in zip(s_o, s_g)) < 1e-12
+    ctx.close()
