@@ -598,54 +598,11 @@ __global__ void k_cluster_bbox(MdgBox B, int nclu, const int *__restrict__ slotA
                          (float)(0.5 * (hi[2] - lo[2])) + 1e-3f, 0.f);
 }
 
-// Exact reference predicate for the unordered pair (i, j): the same FP64
-// expression list.c evaluates for whichever builder the run uses, plus the
-// frozen and exclusion tests.  The value does not depend on the order of
-// i and j (negation is exact, nint and the cell shift are odd).
-__device__ inline bool ref_pair_pred(const MdgParams &P, const MdgBox &B, int keyLink, int nx,
-                                     int ny, int nz, int i, int j, const double *__restrict__ x,
-                                     const double *__restrict__ y, const double *__restrict__ z,
-                                     const double *__restrict__ xu, const double *__restrict__ yu,
-                                     const double *__restrict__ zu, const int *__restrict__ cellOf,
-                                     const int *__restrict__ frozen, const int *__restrict__ exOff,
-                                     const int *__restrict__ exLst)
-{
-#pragma clang fp contract(off)
-    double r2;
-    if (keyLink) {
-        int ci = cellOf[i], cj = cellOf[j];
-        int ix = ci % nx, iy = (ci / nx) % ny, iz = ci / (nx * ny);
-        int jx = cj % nx, jy = (cj / nx) % ny, jz = cj / (nx * ny);
-        int d[3] = {jx - ix, jy - iy, jz - iz};
-        int nn[3] = {nx, ny, nz};
-        double c[3];
-        for (int k = 0; k < 3; k++) {
-            if (d[k] == 0 || d[k] == 1 || d[k] == -1) c[k] = 0.;
-            else if (d[k] == -(nn[k] - 1)) c[k] = 1.;     // j's cell wrapped past the top
-            else if (d[k] == nn[k] - 1) c[k] = -1.;       // j's cell wrapped past the bottom
-            else return false;                             // not neighbouring cells
-        }
-        double xt = xu[j] - xu[i] + c[0];
-        double yt = yu[j] - yu[i] + c[1];
-        double zt = zu[j] - zu[i] + c[2];
-        double xd = xt * B.a1 + yt * B.b1 + zt * B.c1;
-        double yd = xt * B.a2 + yt * B.b2 + zt * B.c2;
-        double zd = xt * B.a3 + yt * B.b3 + zt * B.c3;
-        r2 = xd * xd + yd * yd + zd * zd;
-    } else {
-        int lo = min(i, j), hi = max(i, j);
-        double dx = x[hi] - x[lo], dy = y[hi] - y[lo], dz = z[hi] - z[lo];
-        r2 = mdg_dist(B, dx, dy, dz);
-    }
-    if (!(r2 <= P.cutnb2)) return false;
-    if (frozen[i] * frozen[j]) return false;
-    // the O(N^2) table keeps a pair at its smaller index only (list.c:882-890);
-    // the link-cell table keeps it at both (list.c:1779-1787)
-    return !mdg_excluded(exOff, exLst, min(i, j), max(i, j));
-}
-
-// ref_pair_pred on slot-ordered copies of the predicate inputs (the same
-// FP64 expressions): atoms ia, ja with predicate coordinates (scaled for
+// Exact reference predicate for an unordered pair: the same FP64 expression
+// list.c evaluates for whichever builder the run uses, plus the frozen and
+// exclusion tests.  The value does not depend on the order of the two (negation
+// is exact, nint and the cell shift are odd).  Inputs are slot-ordered copies:
+// atoms ia, ja with predicate coordinates (scaled for
 // link cells, else positions) and link cells ci, cj.  The exclusion table
 // is searched only when |ia - ja| is within the largest excluded span, and
 // frozen flags only when the system has frozen atoms.
@@ -749,6 +706,75 @@ struct ColGrid {
     int ncx, ncy, rx, ry;        // columns per row / rows, reach in each
 };
 
+// Where a wave's found entries (J, mask) go: room for cap of them.
+struct PairSink {
+    int *J;
+    unsigned long long *mask;
+    int cap;
+};
+
+// The 64 exact pair predicates of i cluster I against each candidate J0 + bit of
+// cm, in order; their slot records are requested CAND_BATCH at a time before the
+// first is tested.
+__device__ __forceinline__ void test_candidates(const MdgParams &P, const MdgBox &B, int keyLink,
+                                                int nx, int ny, int nz, int I, int J0,
+                                                unsigned long long cm, const double4 &pi,
+                                                const double4 *__restrict__ pk, bool hasFrozen,
+                                                const int *__restrict__ frozen,
+                                                const int *__restrict__ exOff,
+                                                const int *__restrict__ exLst, int exSpan,
+                                                const PairSink &S, int &found)
+{
+    const int lane = threadIdx.x & 63;
+    const int a = lane & 7, b = lane >> 3;   // i, j atom: mask bit = lane = 8 j + i
+    const int iat = __double2hiint(pi.w), cli = __double2loint(pi.w);
+    while (cm) {
+        int src[CAND_BATCH];
+        int cnt = 0;
+#pragma unroll
+        for (int t = 0; t < CAND_BATCH; t++) {
+            src[t] = cm ? __ffsll((long long)cm) - 1 : 0;
+            if (cm) {
+                cm &= cm - 1;
+                cnt++;
+            }
+        }
+        double4 pj[CAND_BATCH];
+#pragma unroll
+        for (int t = 0; t < CAND_BATCH; t++)
+            pj[t] = pk[(J0 + (t < cnt ? src[t] : src[0])) * MDG_CL + b];
+#pragma unroll
+        for (int t = 0; t < CAND_BATCH; t++) {
+            if (t >= cnt) break;
+            const int Jc = J0 + src[t];
+            const int jat = __double2hiint(pj[t].w), clj = __double2loint(pj[t].w);
+            bool pr = false;
+            if (iat >= 0 && jat >= 0 && (Jc != I || a < b))
+                pr = ref_pair_pred_slot(P, B, keyLink, nx, ny, nz, iat, jat, pi.x, pi.y, pi.z, cli,
+                                        pj[t].x, pj[t].y, pj[t].z, clj, hasFrozen, frozen, exOff,
+                                        exLst, exSpan);
+            const unsigned long long m = __ballot(pr);
+            if (m) {
+                if (found < S.cap && lane == 0) {
+                    S.J[found] = Jc;
+                    S.mask[found] = m;
+                }
+                found++;
+            }
+        }
+    }
+}
+
+// SPLIT wavefronts share an I cluster's column rows (in order, so their finds
+// joined in order are the one-wave list).  A box of few clusters has fewer
+// wavefronts than the chip has SIMDs and is bound by one cluster's chain of
+// candidates; a large one fills the chip with one wavefront a cluster and is bound
+// by the predicate's FP64 issue.  Four wavefronts against one: 648 atoms (about 100
+// clusters) 16 : 46 us, 3,000 59 : 148, 30,000 (3,900 clusters) 194 : 196.
+#define SPLIT_NCLU 4096           // clusters up to which four wavefronts share one
+#define SPLIT_CAP 160            // finds a sharing wavefront keeps (else one wave redoes the cluster)
+
+template <int SPLIT>
 __global__ void __launch_bounds__(256)
 k_cluster_pairs(MdgParams P, MdgBox B, int keyLink, int nx, int ny, int nz, int nclu,
                 const float4 *__restrict__ bb,
@@ -758,8 +784,8 @@ k_cluster_pairs(MdgParams P, MdgBox B, int keyLink, int nx, int ny, int nz, int 
                 int *__restrict__ tmpCnt, int *__restrict__ tmpJ,
                 unsigned long long *__restrict__ tmpMask, int *__restrict__ ctrl, ColGrid CG)
 {
-    const int lane = threadIdx.x & 63;
-    const int I = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int I = SPLIT > 1 ? blockIdx.x : blockIdx.x * 4 + wv;
     if (I >= nclu) return;
     const int colI = CG.cluCol[I];
     if (colI < 0) {
@@ -769,92 +795,83 @@ k_cluster_pairs(MdgParams P, MdgBox B, int keyLink, int nx, int ny, int nz, int 
     const float4 ci = bb[I], hi = bbh[I];
     const float L0 = (float)B.a1, L1 = (float)B.b2, L2 = (float)B.c3;
     const float rl = (float)(P.cutOff + P.delr) + 0.01f;
-    const int a = lane & 7, b = lane >> 3;   // i, j atom: mask bit = lane = 8 j + i
-    const int si = I * MDG_CL + a;
-    const double4 pi = pk[si];
-    const int iat = __double2hiint(pi.w), cli = __double2loint(pi.w);
-    const double xi = pi.x, yi = pi.y, zi = pi.z;
+    const double4 pi = pk[I * MDG_CL + (lane & 7)];
     const int cx = colI % CG.ncx, cy = colI / CG.ncx;
     // rows: all of them once when the reach covers the box, else cy +- ry
     const bool allRows = 2 * CG.ry + 1 >= CG.ncy, allCols = 2 * CG.rx + 1 >= CG.ncx;
     const int nrow = allRows ? CG.ncy : 2 * CG.ry + 1;
-    int found = 0;
-    for (int rr = 0; rr < nrow; rr++) {
-        const int row = allRows ? rr : (cy - CG.ry + rr + CG.ncy) % CG.ncy;
-        // the row's columns in reach as up to two index ranges [lo, hi)
-        int rlo[2], rhi[2], nr = 1;
-        if (allCols) {
-            rlo[0] = 0;
-            rhi[0] = CG.ncx;
-        } else {
-            const int lo = cx - CG.rx, hc = cx + CG.rx + 1;
-            if (lo < 0) {
-                rlo[0] = lo + CG.ncx; rhi[0] = CG.ncx; rlo[1] = 0; rhi[1] = hc; nr = 2;
-            } else if (hc > CG.ncx) {
-                rlo[0] = lo; rhi[0] = CG.ncx; rlo[1] = 0; rhi[1] = hc - CG.ncx; nr = 2;
+    auto search = [&](int r0, int r1, const PairSink &S) {
+        int found = 0;
+        for (int rr = r0; rr < r1; rr++) {
+            const int row = allRows ? rr : (cy - CG.ry + rr + CG.ncy) % CG.ncy;
+            // the row's columns in reach as up to two index ranges [lo, hi)
+            int rlo[2], rhi[2], nr = 1;
+            if (allCols) {
+                rlo[0] = 0;
+                rhi[0] = CG.ncx;
             } else {
-                rlo[0] = lo; rhi[0] = hc;
-            }
-        }
-        for (int q = 0; q < nr; q++) {
-            const int j0 = max(I, CG.colSlot[row * CG.ncx + rlo[q]] / MDG_CL);
-            const int j1 = CG.colSlot[row * CG.ncx + rhi[q]] / MDG_CL;
-            for (int J0 = j0; J0 < j1; J0 += 64) {
-                const int J = J0 + lane;
-                bool cand = false;
-                if (J < j1) {
-                    const float4 cj = bb[J], hj = bbh[J];
-                    float dx = cj.x - ci.x, dy = cj.y - ci.y, dz = cj.z - ci.z;
-                    if (B.type == 1 || B.type == 2) {
-                        dx -= L0 * rintf(dx / L0);
-                        dy -= L1 * rintf(dy / L1);
-                        dz -= L2 * rintf(dz / L2);
-                    }
-                    dx = fmaxf(fabsf(dx) - hi.x - hj.x, 0.f);
-                    dy = fmaxf(fabsf(dy) - hi.y - hj.y, 0.f);
-                    dz = fmaxf(fabsf(dz) - hi.z - hj.z, 0.f);
-                    cand = B.type == 3 || (dx * dx + dy * dy + dz * dz <= rl * rl);
+                const int lo = cx - CG.rx, hc = cx + CG.rx + 1;
+                if (lo < 0) {
+                    rlo[0] = lo + CG.ncx; rhi[0] = CG.ncx; rlo[1] = 0; rhi[1] = hc; nr = 2;
+                } else if (hc > CG.ncx) {
+                    rlo[0] = lo; rhi[0] = CG.ncx; rlo[1] = 0; rhi[1] = hc - CG.ncx; nr = 2;
+                } else {
+                    rlo[0] = lo; rhi[0] = hc;
                 }
-                unsigned long long cm = __ballot(cand);
-                // candidates in order, CAND_BATCH at a time: their slot
-                // records are all requested before the first is tested
-                while (cm) {
-                    int src[CAND_BATCH];
-                    int cnt = 0;
-#pragma unroll
-                    for (int t = 0; t < CAND_BATCH; t++) {
-                        src[t] = cm ? __ffsll((long long)cm) - 1 : 0;
-                        if (cm) {
-                            cm &= cm - 1;
-                            cnt++;
+            }
+            for (int q = 0; q < nr; q++) {
+                const int j0 = max(I, CG.colSlot[row * CG.ncx + rlo[q]] / MDG_CL);
+                const int j1 = CG.colSlot[row * CG.ncx + rhi[q]] / MDG_CL;
+                for (int J0 = j0; J0 < j1; J0 += 64) {
+                    const int J = J0 + lane;
+                    bool cand = false;
+                    if (J < j1) {
+                        const float4 cj = bb[J], hj = bbh[J];
+                        float dx = cj.x - ci.x, dy = cj.y - ci.y, dz = cj.z - ci.z;
+                        if (B.type == 1 || B.type == 2) {
+                            dx -= L0 * rintf(dx / L0);
+                            dy -= L1 * rintf(dy / L1);
+                            dz -= L2 * rintf(dz / L2);
                         }
+                        dx = fmaxf(fabsf(dx) - hi.x - hj.x, 0.f);
+                        dy = fmaxf(fabsf(dy) - hi.y - hj.y, 0.f);
+                        dz = fmaxf(fabsf(dz) - hi.z - hj.z, 0.f);
+                        cand = B.type == 3 || (dx * dx + dy * dy + dz * dz <= rl * rl);
                     }
-                    double4 pj[CAND_BATCH];
-#pragma unroll
-                    for (int t = 0; t < CAND_BATCH; t++)
-                        pj[t] = pk[(J0 + (t < cnt ? src[t] : src[0])) * MDG_CL + b];
-#pragma unroll
-                    for (int t = 0; t < CAND_BATCH; t++) {
-                        if (t >= cnt) break;
-                        const int Jc = J0 + src[t];
-                        const int jat = __double2hiint(pj[t].w), clj = __double2loint(pj[t].w);
-                        bool pr = false;
-                        if (iat >= 0 && jat >= 0 && (Jc != I || a < b))
-                            pr = ref_pair_pred_slot(P, B, keyLink, nx, ny, nz, iat, jat, xi, yi,
-                                                    zi, cli, pj[t].x, pj[t].y, pj[t].z, clj,
-                                                    hasFrozen, frozen, exOff, exLst, exSpan);
-                        const unsigned long long m = __ballot(pr);
-                        if (m) {
-                            if (found < kmax && lane == 0) {
-                                tmpJ[(long)I * kmax + found] = Jc;
-                                tmpMask[(long)I * kmax + found] = m;
-                            }
-                            found++;
-                        }
-                    }
+                    test_candidates(P, B, keyLink, nx, ny, nz, I, J0, __ballot(cand), pi, pk,
+                                    hasFrozen, frozen, exOff, exLst, exSpan, S, found);
                 }
             }
         }
+        return found;
+    };
+    const PairSink out = {tmpJ + (long)I * kmax, tmpMask + (long)I * kmax, kmax};
+    int found;
+    if (SPLIT > 1) {
+        __shared__ int sJ[SPLIT][SPLIT_CAP], sn[SPLIT];
+        __shared__ unsigned long long sM[SPLIT][SPLIT_CAP];
+        const int mine = search(wv * nrow / SPLIT, (wv + 1) * nrow / SPLIT,
+                                PairSink{sJ[wv], sM[wv], SPLIT_CAP});
+        if (lane == 0) sn[wv] = mine;
+        __syncthreads();
+        int base = 0, over = 0;
+        found = 0;
+        for (int w = 0; w < SPLIT; w++) {
+            if (w < wv) base += sn[w];
+            found += sn[w];
+            over |= sn[w] > SPLIT_CAP;
+        }
+        if (over) {
+            if (wv == 0) search(0, nrow, out);
+        } else {
+            for (int k = lane; k < mine && base + k < kmax; k += 64) {
+                out.J[base + k] = sJ[wv][k];
+                out.mask[base + k] = sM[wv][k];
+            }
+        }
+        if (wv > 0) return;
+    } else {
+        found = search(0, nrow, out);
     }
     if (lane == 0) {
         tmpCnt[I] = min(found, kmax);
@@ -1110,7 +1127,9 @@ int mdg_build_cluster_list(mdg_ctx *ctx)
         CG.rx = (int)(rl / (ctx->B.pa / C.nfx)) + 1;
         CG.ry = (int)(rl / (ctx->B.pb / C.nfy)) + 1;
     }
-    hipLaunchKernelGGL(k_cluster_pairs, dim3(nblk(nclu, 4)), dim3(256), 0, ctx->stream, ctx->P,
+    const bool split = nclu <= SPLIT_NCLU;
+    hipLaunchKernelGGL(split ? k_cluster_pairs<4> : k_cluster_pairs<1>,
+                       dim3(split ? nclu : nblk(nclu, 4)), dim3(256), 0, ctx->stream, ctx->P,
                        ctx->B, ctx->keyLink, ctx->nlc[0], ctx->nlc[1], ctx->nlc[2], nclu,
                        C.bb, C.bbh, C.pk, ctx->hasFrozen,
                        ctx->frozen, ctx->exOff, ctx->exLst, ctx->exSpan, C.kmax, C.tmpCnt, C.tmpJ,
@@ -1197,15 +1216,17 @@ __global__ void k_b_cluster_bbox(const MdgBox *__restrict__ boxes, const int *__
 
 // k_cluster_pairs for a batch: J runs over I's own replica only, with that
 // replica's box, and the O(N^2) predicate of verlet_list (list.c:896-1040).
+// From slot records and four candidates ahead, as there: 256 replicas of 216 to
+// 400 waters 410 us, with the atoms' coordinates, frozen flags and exclusions
+// gathered per candidate 1,177.
 __global__ void __launch_bounds__(256)
 k_b_cluster_pairs(MdgParams P, const MdgBox *__restrict__ boxes, const int *__restrict__ crep,
-                  const int *__restrict__ cluStart, int nclu, const int *__restrict__ slotAtom,
-                  const float4 *__restrict__ bb, const float4 *__restrict__ bbh,
-                  const double *__restrict__ x, const double *__restrict__ y,
-                  const double *__restrict__ z, const int *__restrict__ frozen,
-                  const int *__restrict__ exOff, const int *__restrict__ exLst, int kmax,
-                  int *__restrict__ tmpCnt, int *__restrict__ tmpJ,
-                  unsigned long long *__restrict__ tmpMask, int *__restrict__ ctrl)
+                  const int *__restrict__ cluStart, int nclu, const float4 *__restrict__ bb,
+                  const float4 *__restrict__ bbh, const double4 *__restrict__ pk, bool hasFrozen,
+                  const int *__restrict__ frozen, const int *__restrict__ exOff,
+                  const int *__restrict__ exLst, int exSpan, int kmax, int *__restrict__ tmpCnt,
+                  int *__restrict__ tmpJ, unsigned long long *__restrict__ tmpMask,
+                  int *__restrict__ ctrl)
 {
     const int lane = threadIdx.x & 63;
     const int I = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
@@ -1215,16 +1236,16 @@ k_b_cluster_pairs(MdgParams P, const MdgBox *__restrict__ boxes, const int *__re
         if (lane == 0) tmpCnt[I] = 0;
         return;
     }
-    const MdgBox &B = boxes[r];
+    const MdgBox &B = boxes[__builtin_amdgcn_readfirstlane(r)];
     const int jend = cluStart[r + 1];
     const float4 ci = bb[I], hi = bbh[I];
     const float L0 = (float)B.a1, L1 = (float)B.b2, L2 = (float)B.c3;
     const float rl = (float)(P.cutOff + P.delr) + 0.01f;
-    const int a = lane & 7, b = lane >> 3;   // i, j atom: mask bit = lane = 8 j + i
-    const int iat = slotAtom[I * MDG_CL + a];
+    const double4 pi = pk[I * MDG_CL + (lane & 7)];
+    const PairSink out = {tmpJ + (long)I * kmax, tmpMask + (long)I * kmax, kmax};
     int found = 0;
     for (int J0 = I; J0 < jend; J0 += 64) {
-        int J = J0 + lane;
+        const int J = J0 + lane;
         bool cand = false;
         if (J < jend) {
             float4 cj = bb[J], hj = bbh[J];
@@ -1237,25 +1258,8 @@ k_b_cluster_pairs(MdgParams P, const MdgBox *__restrict__ boxes, const int *__re
             dz = fmaxf(fabsf(dz) - hi.z - hj.z, 0.f);
             cand = dx * dx + dy * dy + dz * dz <= rl * rl;
         }
-        unsigned long long cm = __ballot(cand);
-        while (cm) {
-            int src = __ffsll((long long)cm) - 1;
-            cm &= cm - 1;
-            int Jc = J0 + src;
-            int jat = slotAtom[Jc * MDG_CL + b];
-            bool pr = false;
-            if (iat >= 0 && jat >= 0 && (Jc != I || a < b))
-                pr = ref_pair_pred(P, B, 0, 0, 0, 0, iat, jat, x, y, z, nullptr, nullptr, nullptr,
-                                   nullptr, frozen, exOff, exLst);
-            unsigned long long m = __ballot(pr);
-            if (m) {
-                if (found < kmax && lane == 0) {
-                    tmpJ[(long)I * kmax + found] = Jc;
-                    tmpMask[(long)I * kmax + found] = m;
-                }
-                found++;
-            }
-        }
+        test_candidates(P, B, 0, 0, 0, 0, I, J0, __ballot(cand), pi, pk, hasFrozen, frozen, exOff,
+                        exLst, exSpan, out, found);
     }
     if (lane == 0) {
         tmpCnt[I] = min(found, kmax);
@@ -1280,6 +1284,7 @@ int mdg_b_build_list(mdg_ctx *ctx)
         HIPCHK(hipMalloc(&C.sortTmp, n * sizeof(int)));
         HIPCHK(hipMalloc(&C.sortKey, n * sizeof(float)));
         HIPCHK(hipMalloc(&C.slotAtom, ((size_t)maxclu * MDG_CL + 64) * sizeof(int)));
+        HIPCHK(hipMalloc(&C.pk, ((size_t)maxclu * MDG_CL + 64) * sizeof(double4)));
         HIPCHK(hipMalloc(&C.atomSlot, n * sizeof(int)));
         HIPCHK(hipMalloc(&C.bb, maxclu * sizeof(float4)));
         HIPCHK(hipMalloc(&C.bbh, maxclu * sizeof(float4)));
@@ -1316,9 +1321,13 @@ int mdg_b_build_list(mdg_ctx *ctx)
     hipLaunchKernelGGL(k_b_cluster_bbox, dim3(nblk(nclu, 128)), dim3(128), 0, ctx->stream, T.boxes,
                        T.arep, nclu, C.slotAtom, ctx->x, ctx->y, ctx->z, C.bb, C.bbh, T.crep);
     LAUNCHCHK();
+    hipLaunchKernelGGL(k_pred_slots, dim3(nblk(nclu * MDG_CL, 256)), dim3(256), 0, ctx->stream,
+                       nclu * MDG_CL, 0, 1, 1, C.slotAtom, ctx->x, ctx->y, ctx->z, ctx->x, ctx->y,
+                       ctx->z, nullptr, C.pk);
+    LAUNCHCHK();
     hipLaunchKernelGGL(k_b_cluster_pairs, dim3(nblk(nclu, 4)), dim3(256), 0, ctx->stream, ctx->P,
-                       T.boxes, T.crep, T.cluStart, nclu, C.slotAtom, C.bb, C.bbh, ctx->x, ctx->y,
-                       ctx->z, ctx->frozen, ctx->exOff, ctx->exLst, C.kmax, C.tmpCnt, C.tmpJ,
+                       T.boxes, T.crep, T.cluStart, nclu, C.bb, C.bbh, C.pk, ctx->listFrozen,
+                       ctx->frozen, ctx->exOff, ctx->exLst, ctx->exSpan, C.kmax, C.tmpCnt, C.tmpJ,
                        C.tmpMask, ctx->ctrl);
     LAUNCHCHK();
     RETCHK(compact_cluster_list(ctx));
