@@ -1217,7 +1217,7 @@ __global__ void k_b_cluster_bbox(const MdgBox *__restrict__ boxes, const int *__
 // k_cluster_pairs for a batch: J runs over I's own replica only, with that
 // replica's box, and the O(N^2) predicate of verlet_list (list.c:896-1040).
 // From slot records and four candidates ahead, as there: 256 replicas of 216 to
-// 400 waters 410 us, with the atoms' coordinates, frozen flags and exclusions
+// 512 waters 410 us, with the atoms' coordinates, frozen flags and exclusions
 // gathered per candidate 1,177.
 __global__ void __launch_bounds__(256)
 k_b_cluster_pairs(MdgParams P, const MdgBox *__restrict__ boxes, const int *__restrict__ crep,
