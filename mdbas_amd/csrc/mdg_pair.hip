@@ -1442,56 +1442,65 @@ int mdg_prune_list(mdg_ctx *ctx)
 //   dE/deps_i += eps_j 4 (s^12 - s^6) S(r)                (and i <-> j)
 //   dE/dsig_i += 4 eps_i eps_j (12 s^11 - 6 s^5) S(r) / r (both atoms)
 // with s = (sig_i + sig_j) / r and S the switch of vdw.c:144-184 (1 below
-// cutOn).  Same wavefront layout as k_pair_fp64; slot sums go to
-// fdx (q), fdy (eps), fdz (sig).
+// cutOn).  Same wavefront layout, loads ahead and functions as k_pair_fp64; slot
+// sums go to fdx (q), fdy (eps), fdz (sig).  FP64 issue; 12,000 atoms 119 us (161
+// with library functions, per-component sums and no loads ahead), 3,000 37.
 __global__ void __launch_bounds__(256) k_adj_cluster(ClusterArgs A)
 {
     const int lane = threadIdx.x & 63;
     const int a = lane & 7, b = lane >> 3;
-    const int bit = lane;
-    const int nch = min(A.chOff[A.nclu], A.maxChunks);
-    for (int W = blockIdx.x * 4 + (threadIdx.x >> 6); W < nch; W += gridDim.x * 4) {
-        const int2 ch = A.chunk[W];
-        const int I = ch.x, e0 = ch.y, e1 = min(min(e0 + A.chunkLen, A.cpOff[I + 1]), A.cap);
+    const int nch = min(mdg_uload(A.chOff, A.nclu), A.maxChunks);
+    for (int W = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); W < nch;
+         W += gridDim.x * 4) {
+        const long ch = mdg_uload((const long *)A.chunk, W);   // int2 (I, e0)
+        const int I = (int)(ch & 0xffffffffl), e0 = (int)(ch >> 32);
+        const int e1 = min(min(e0 + A.chunkLen, mdg_uload(A.cpOff, I + 1)), A.cap);
+        if (e0 >= e1) continue;   // only after a flagged list overflow
         const int si = I * MDG_CL + a;
-        const double xi = A.sx[si], yi = A.sy[si], zi = A.sz[si];
-        const double qi = A.sq[si], ei = A.seps[si], gi = A.ssig[si];
+        const Fp64J pi = fp64_load(A, si);
         double gqi = 0., gei = 0., gsi = 0.;
+        int J = mdg_uload(A.cpJ, e0);
+        unsigned long long m = mdg_uload(A.cpMask, e0);
+        Fp64J pj = fp64_load(A, J * MDG_CL + b);
         for (int e = e0; e < e1; e++) {
-            const int J = A.cpJ[e];
-            const unsigned long long m = A.cpMask[e];
-            const int sj = J * MDG_CL + b;
-            double dx = A.sx[sj] - xi, dy = A.sy[sj] - yi, dz = A.sz[sj] - zi;
-            const double r2 = mdg_dist(A.B, dx, dy, dz);
-            double gqj = 0., gej = 0., gsj = 0.;
-            if (((m >> bit) & 1ull) && r2 <= A.P.cutOff2) {
-                const double r = sqrt(r2), rt = 1. / r;
-                const double qj = A.sq[sj], ej = A.seps[sj];
-                const double ec = A.P.chargeConst * erfc(A.P.alpha * r) * rt;
-                gqi += qj * ec;
-                gqj = qi * ec;
-                const double s = (gi + A.ssig[sj]) * rt, s2 = s * s, s6 = s2 * s2 * s2;
-                const double s12 = s6 * s6, s5 = s2 * s2 * s, s11 = s5 * s6;
-                double S = 1.;
-                if (r2 > A.P.cutOn2) {
-                    const double sw = A.P.cutOff2 - r2;
-                    S = sw * sw * (A.P.cutOff2 + 2. * r2 - 3. * A.P.cutOn2) * A.P.switch2;
+            const int en = min(e + 1, e1 - 1);
+            const int Jn = mdg_uload(A.cpJ, en);
+            const unsigned long long mn = mdg_uload(A.cpMask, en);
+            const Fp64J pn = fp64_load(A, Jn * MDG_CL + b);
+            double dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+            const double r2 = fp64_dist(A.B, dx, dy, dz);
+            const unsigned long long inm = m & __builtin_amdgcn_ballot_w64(r2 <= A.P.cutOff2);
+            // an entry with no pair inside the cutoff adds only exact zeros
+            if (inm != 0) {
+                double gqj = 0., gej = 0., gsj = 0.;
+                if (__builtin_amdgcn_inverse_ballot_w64(inm)) {
+                    double r, ez;
+                    const double rt = mdg_rsqrt64(r2, r);
+                    const double ec = A.P.chargeConst * mdg_erfc64(A.P.alpha * r, ez) * rt;
+                    gqi += pj.q * ec;
+                    gqj = pi.q * ec;
+                    const double s = (pi.g + pj.g) * rt, s2 = s * s, s6 = s2 * s2 * s2;
+                    const double s12 = s6 * s6, s5 = s2 * s2 * s, s11 = s5 * s6;
+                    double S = 1.;
+                    if (r2 > A.P.cutOn2) {
+                        const double sw = A.P.cutOff2 - r2;
+                        S = sw * sw * (A.P.cutOff2 + 2. * r2 - 3. * A.P.cutOn2) * A.P.switch2;
+                    }
+                    const double lj = 4. * (s12 - s6) * S;
+                    gei += pj.e * lj;
+                    gej = pi.e * lj;
+                    const double gs = 4. * pi.e * pj.e * (12. * s11 - 6. * s5) * rt * S;
+                    gsi += gs;
+                    gsj = gs;
                 }
-                const double lj = 4. * (s12 - s6) * S;
-                gei += ej * lj;
-                gej = ei * lj;
-                const double gs = 4. * ei * ej * (12. * s11 - 6. * s5) * rt * S;
-                gsi += gs;
-                gsj = gs;
+                const double k = dpp_rs8d(gqj, gej, gsj, a);
+                const int sj = J * MDG_CL + b;
+                if ((a & 1) == 0 && a < 6 && k != 0.)
+                    atomicAdd(a == 0 ? &A.fdx[sj] : (a == 2 ? &A.fdy[sj] : &A.fdz[sj]), k);
             }
-            gqj = dpp_sum8(gqj);
-            gej = dpp_sum8(gej);
-            gsj = dpp_sum8(gsj);
-            if (a == 0) {
-                if (gqj != 0.) atomicAdd(&A.fdx[sj], gqj);
-                if (gej != 0.) atomicAdd(&A.fdy[sj], gej);
-                if (gsj != 0.) atomicAdd(&A.fdz[sj], gsj);
-            }
+            J = Jn;
+            m = mn;
+            pj = pn;
         }
         for (int o = 8; o < 64; o <<= 1) {
             gqi += __shfl_xor(gqi, o, 64);
