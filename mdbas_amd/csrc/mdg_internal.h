@@ -623,11 +623,13 @@ void mdg_params_from(const MDG_CTRL *ctrl, const MDG_PARAM *p, MdgParams &P);
 // into part, mdg_ref64_blocks(n) rows.  A block takes mdg_ref64_group(n) rows
 // of the list: whole rounds of the 256 CUs (a block fills one) with at most 32
 // rows a block, beyond which a group's distinct j outgrow its LDS table, and at
-// least 4, below which rows would share too few j to collect.
+// least 4, below which rows would share too few j to collect.  Above 1.4 million
+// atoms the groups grow instead of their number: the partials have one region
+// of epart.
 inline int mdg_ref64_group(int n)
 {
     const int rounds = nblk(n, 256 * 32);
-    return std::max(nblk(n, 256 * rounds), 4);
+    return std::max({nblk(n, 256 * rounds), 4, nblk(n, PART_R / 6)});
 }
 inline int mdg_ref64_blocks(int n) { return nblk(n, mdg_ref64_group(n)); }
 int mdg_ref_pack_launch(hipStream_t stream, int n, const double *x, const double *y,
