@@ -827,13 +827,20 @@ static void put_xyzq(mdg_ctx *ctx, MdgXfer &X, const double *x, const double *y,
     if (sig) X.put(ctx->sig, sig, n);
 }
 
-// Forces to or from the device (null on the way up: zeros).
+// Forces to or from the device.
 static void put_forces(mdg_ctx *ctx, MdgXfer &X, const double *fx, const double *fy,
                        const double *fz)
 {
     X.put(ctx->fx, fx, ctx->n);
     X.put(ctx->fy, fy, ctx->n);
     X.put(ctx->fz, fz, ctx->n);
+}
+
+static void zero_forces(mdg_ctx *ctx, MdgXfer &X)
+{
+    X.zero(ctx->fx, ctx->n);
+    X.zero(ctx->fy, ctx->n);
+    X.zero(ctx->fz, ctx->n);
 }
 
 // ---------------------------------------------------------------- drop-in: makelist
@@ -996,12 +1003,12 @@ extern "C" int mdg_spme_energy(mdg_ctx *ctx, MDG_PARAM *param, MDG_EWALD *ewald,
 // energy.c:450-643 on the device: uploads positions, parameters, list and
 // exclusions and forces fx (the caller's +=), runs SPME (keyEwald 2), the
 // real-space pairs and the excluded-pair correction into ctx->fx..; the
-// forces and the sums (scal) stay on the device.  fx null: from zero.
+// forces and the sums (scal) stay on the device.  fromZero: fx.. are not read.
 static int ewald_on_device(mdg_ctx *ctx, const MDG_CTRL *ctrl, const double *x, const double *y,
                            const double *z, const double *fx, const double *fy, const double *fz,
                            const double *q, const double *eps, const double *sig,
                            const int *neighList, const int *neighPair, const int *neighOrder,
-                           int **exclList, const int *exclPair)
+                           int **exclList, const int *exclPair, bool fromZero)
 {
     if (ctrl->keyEwald == 1) {
         ctx->err = "classic k-space Ewald (keyEwald 1) is not on this path";
@@ -1011,7 +1018,8 @@ static int ewald_on_device(mdg_ctx *ctx, const MDG_CTRL *ctrl, const double *x, 
     MdgXfer X(true);
     std::vector<long> off;
     put_xyzq(ctx, X, x, y, z, q, eps, sig);
-    put_forces(ctx, X, fx, fy, fz);
+    if (fromZero) zero_forces(ctx, X);
+    else put_forces(ctx, X, fx, fy, fz);
     RETCHK(upload_ref_list(ctx, X, off, neighList, neighPair, neighOrder));
     RETCHK(exclusions_from_args(ctx, exclList, exclPair));
     RETCHK(X.up(ctx));
@@ -1043,7 +1051,7 @@ static int nonbond_on_device(mdg_ctx *ctx, const MDG_CTRL *ctrl, const double *x
                              const double *z, const double *fx, const double *fy,
                              const double *fz, const double *q, const double *eps,
                              const double *sig, const int *neighList, const int *neighPair,
-                             const int *neighOrder)
+                             const int *neighOrder, bool fromZero)
 {
     // energy.c:45-65: FULL and NOELEC evaluate no electrostatics
     int et = ctrl->elecType;
@@ -1053,7 +1061,8 @@ static int nonbond_on_device(mdg_ctx *ctx, const MDG_CTRL *ctrl, const double *x
     MdgXfer X(true);
     std::vector<long> off;
     put_xyzq(ctx, X, x, y, z, q, eps, sig);
-    put_forces(ctx, X, fx, fy, fz);
+    if (fromZero) zero_forces(ctx, X);
+    else put_forces(ctx, X, fx, fy, fz);
     RETCHK(upload_ref_list(ctx, X, off, neighList, neighPair, neighOrder));
     RETCHK(X.up(ctx));
     return mdg_pair_ref64(ctx, et, ctx->fx, ctx->fy, ctx->fz, ctx->rl.neighList, ctx->rl.off,
@@ -1071,7 +1080,7 @@ extern "C" int mdg_ewald_energy(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, 
     if (!ctx || !ctrl || !ener || !x || !fx || !q || !neighPair || !neighOrder) return MDG_EARG;
     if (box) RETCHK(mdg_refresh_box(ctx, box));
     RETCHK(ewald_on_device(ctx, ctrl, x, y, z, fx, fy, fz, q, eps, sig, neighList, neighPair,
-                           neighOrder, exclList, exclPair));
+                           neighOrder, exclList, exclPair, false));
     double e[4], h[S_COUNT];
     MdgXfer D(false);
     D.put(ctx->scal, h, S_COUNT);
@@ -1097,7 +1106,7 @@ extern "C" int mdg_nonbond_energy(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param
     if (!ctx || !ctrl || !ener || !x || !fx || !q || !neighPair || !neighOrder) return MDG_EARG;
     if (box) RETCHK(mdg_refresh_box(ctx, box));
     RETCHK(nonbond_on_device(ctx, ctrl, x, y, z, fx, fy, fz, q, eps, sig, neighList, neighPair,
-                             neighOrder));
+                             neighOrder, false));
     double h[S_COUNT];
     MdgXfer D(false);
     D.put(ctx->scal, h, S_COUNT);
@@ -1142,10 +1151,10 @@ extern "C" int mdg_energy(mdg_ctx *ctx, MDG_CTRL *ctrl, MDG_PARAM *param, MDG_EN
     // forces), each followed by its 1-4 pairs when keyNb14 is set
     if (ctrl->keyEwald != 0)
         RETCHK(ewald_on_device(ctx, ctrl, x, y, z, nullptr, nullptr, nullptr, q, eps, sig,
-                               neighList, neighPair, neighOrder, exclList, exclPair));
+                               neighList, neighPair, neighOrder, exclList, exclPair, true));
     else
         RETCHK(nonbond_on_device(ctx, ctrl, x, y, z, nullptr, nullptr, nullptr, q, eps, sig,
-                                 neighList, neighPair, neighOrder));
+                                 neighList, neighPair, neighOrder, true));
     // energy.c:157-189: 1-4 pairs, bonds, angles, Urey-Bradley, dihedrals,
     // impropers, all in one device kernel
     MdgBonded &D = ctx->bd;

@@ -213,16 +213,20 @@ struct MdgXferTab {
 };
 struct MdgXfer {
     explicit MdgXfer(bool toDevice) : in(toDevice) {}
-    void add(void *dev, void *host, size_t bytes);
+    // a host array to or from the device; one that is missing fails up or fetch
     template <typename T> void put(T *dev, const T *host, size_t cnt)
     {
+        missing |= cnt && !host;
         add(dev, const_cast<T *>(host), cnt * sizeof(T));
     }
+    // a device array to clear, on the way up
+    template <typename T> void zero(T *dev, size_t cnt) { add(dev, nullptr, cnt * sizeof(T)); }
     int up(struct mdg_ctx *ctx);
     int fetch(struct mdg_ctx *ctx, int nfirst);
     int deliver(struct mdg_ctx *ctx);
 
   private:
+    void add(void *dev, void *host, size_t bytes);
     int prepare(struct mdg_ctx *ctx);
     int launch(struct mdg_ctx *ctx);
     struct {
@@ -231,7 +235,7 @@ struct MdgXfer {
     } seg[MDG_XFER_SEGS];
     int n = 0, first = 0;
     size_t total = 0;
-    bool in, full = false, packed = false;
+    bool in, full = false, missing = false, packed = false;
     char *buf = nullptr;
 };
 

@@ -56,6 +56,10 @@ int MdgXfer::prepare(mdg_ctx *ctx)
         ctx->err = "too many arrays in one transfer";
         return MDG_EARG;
     }
+    if (missing) {
+        ctx->err = "a host array of the call is missing";
+        return MDG_EARG;
+    }
     packed = total <= XFER_MAX;
     for (int k = 0; k < n; k++)
         if (((uintptr_t)seg[k].dev & 15) || (seg[k].bytes & 3) || seg[k].bytes > XFER_MAX)
@@ -84,8 +88,8 @@ int MdgXfer::launch(mdg_ctx *ctx)
     return MDG_OK;
 }
 
-// Host arrays (null: zeros) to the device, in stream order; the host arrays are
-// free again when it returns.
+// Host arrays (and cleared ones) to the device, in stream order; the host arrays
+// are free again when it returns.
 int MdgXfer::up(mdg_ctx *ctx)
 {
     if (n == 0) return MDG_OK;

@@ -134,3 +134,47 @@ def test_dropin_transfer_sizes(nw):
         ctx.vv_integrate(stage, *s_g, f_o.copy())
         assert max(np.abs(a - b).max() for a, b in zip(s_o, s_g)) < 1e-12
     ctx.close()
+
+
+# A drop-in call without one of its arrays is refused, and the context computes
+# the same afterwards.
+def test_dropin_missing_arrays():
+    wb = water(43, 3.4, 0.4)
+    ctx = M.Context(wb)
+    x, y, z = wb.x.copy(), wb.y.copy(), wb.z.copy()
+    lists = ctx.makelist(x, y, z)[:3]
+    v = [wb.vx.copy(), wb.vy.copy(), wb.vz.copy()]
+    f0 = ctx.energy(x, y, z, *lists)[0]
+    g = M.P
+    e, s, d = M.MDG_ENERGY(), np.zeros(6), C.c_double(0)
+    L, h, by = ctx.L, ctx.h, C.byref
+    el, ep = ctx._excl
+
+    def refused(name, fn, head, arrays, tail):
+        for k in range(len(arrays)):
+            print(name, "without array", k, flush=True)
+            got = [g(a.copy()) for a in arrays]
+            got[k] = None
+            assert fn(h, *head, *got, *tail) != 0, (name, k)
+
+    pos, force = [x, y, z], [np.zeros(wb.n)] * 3
+    par, nl = [wb.q, wb.eps, wb.sig], [g(a) for a in lists]
+    refused("spme", L.mdg_spme_energy, [by(ctx.param), by(ctx.ewald), by(ctx.pbc)],
+            pos + force + [wb.q], [g(s), by(d), by(d)])
+    refused("ewald", L.mdg_ewald_energy,
+            [by(ctx.ctrl), by(ctx.param), by(e), by(ctx.ewald), by(ctx.pbc)], pos + force,
+            [g(a) for a in par] + nl + [el, ep])
+    refused("nonbond", L.mdg_nonbond_energy, [by(ctx.ctrl), by(ctx.param), by(e), by(ctx.pbc)],
+            pos + force, [g(a) for a in par] + nl)
+    head = [by(ctx.ctrl), by(ctx.param), by(e), by(ctx.ewald), by(ctx.pbc), by(ctx.neigh)]
+    none = [None] * 5
+    tail = [g(a) for a in par] + [None, None, g(wb.frozen)] + nl + [None, el, ep]
+    vel = [g(a) for a in v]
+    refused("energy positions", L.mdg_energy, head + none, pos,
+            vel + [g(a) for a in force] + tail)
+    refused("energy forces", L.mdg_energy, head + none + [g(a) for a in pos] + vel, force, tail)
+    refused("vv", L.mdg_vv_integrate,
+            [by(ctx.ctrl), by(ctx.param), by(e), by(ctx.pbc), None, ctx.cons],
+            pos + v + list(f0) + [wb.mass, wb.rmass], [g(wb.nAtConst), 2])
+    assert np.allclose(ctx.energy(x, y, z, *lists)[0], f0, rtol=1e-12, atol=1e-9)
+    ctx.close()
