@@ -486,6 +486,14 @@ __host__ __device__ inline int mdg_nint(double x)
     return x >= 0. ? (int)(x + 0.5) : (int)(x - 0.5);
 }
 
+// mdg_nint without the conversions, for the pair kernels: the same value
+// (rint's ties to even are not: half an edge takes the other image).
+__device__ __forceinline__ double mdg_nintd(double x)
+{
+#pragma clang fp contract(off)
+    return trunc(x + copysign(0.5, x));
+}
+
 // utils.c:38-80 (dist): minimum image of d in place, |d|^2 as
 // (dx^2 + dy^2) + dz^2 without contraction.
 __host__ __device__ inline double mdg_dist(const MdgBox &b, double &dx, double &dy, double &dz)

@@ -94,22 +94,20 @@ __global__ void k_ref_pack(int n, const double *__restrict__ x, const double *__
     at[i].s = make_double4(eps[i], sig[i], 0., 0.);
 }
 
-// Minimum image and r^2 as mdg_dist forms them; the image index is rounded by
-// rint, which differs from the reference's nint only where |d| is within a
-// rounding of half an edge.
+// mdg_dist with the image index rounded in the FP64 unit.
 __device__ __forceinline__ double ref_dist(const MdgBox &b, double &dx, double &dy, double &dz)
 {
 #pragma clang fp contract(off)
     if (b.type == 1) {
-        dx -= b.a1 * rint(dx * b.u1);
-        dy -= b.a1 * rint(dy * b.u1);
-        dz -= b.a1 * rint(dz * b.u1);
+        dx -= b.a1 * mdg_nintd(dx * b.u1);
+        dy -= b.a1 * mdg_nintd(dy * b.u1);
+        dz -= b.a1 * mdg_nintd(dz * b.u1);
         return dx * dx + dy * dy + dz * dz;
     }
     if (b.type == 2) {
-        dx -= b.a1 * rint(dx * b.u1);
-        dy -= b.b2 * rint(dy * b.v2);
-        dz -= b.c3 * rint(dz * b.w3);
+        dx -= b.a1 * mdg_nintd(dx * b.u1);
+        dy -= b.b2 * mdg_nintd(dy * b.v2);
+        dz -= b.c3 * mdg_nintd(dz * b.w3);
         return dx * dx + dy * dy + dz * dz;
     }
     return mdg_dist(b, dx, dy, dz);
@@ -503,8 +501,8 @@ __device__ __forceinline__ Fp64J fp64_load(const ClusterArgs &A, int sj)
     return {A.sx[sj], A.sy[sj], A.sz[sj], A.sq[sj], A.seps[sj], A.ssig[sj]};
 }
 
-// Minimum image and r^2 as mdg_dist forms them, the image index rounded by
-// rint (see mx_ref_r2: the same for every pair inside the cutoff).
+// mdg_dist with the image index rounded in the FP64 unit, one form for both
+// rectangular boxes.
 __device__ __forceinline__ double fp64_dist(const MdgBox &b, double &dx, double &dy, double &dz)
 {
 #pragma clang fp contract(off)
@@ -512,9 +510,9 @@ __device__ __forceinline__ double fp64_dist(const MdgBox &b, double &dx, double 
     const double L1 = b.type == 1 ? b.a1 : b.b2, L2 = b.type == 1 ? b.a1 : b.c3;
     const double i1 = b.type == 1 ? b.u1 : b.v2, i2 = b.type == 1 ? b.u1 : b.w3;
     if (b.type != 0) {
-        dx -= b.a1 * rint(dx * b.u1);
-        dy -= L1 * rint(dy * i1);
-        dz -= L2 * rint(dz * i2);
+        dx -= b.a1 * mdg_nintd(dx * b.u1);
+        dy -= L1 * mdg_nintd(dy * i1);
+        dz -= L2 * mdg_nintd(dz * i2);
     }
     return dx * dx + dy * dy + dz * dz;
 }

@@ -178,3 +178,35 @@ def test_dropin_missing_arrays():
             pos + v + list(f0) + [wb.mass, wb.rmass], [g(wb.nAtConst), 2])
     assert np.allclose(ctx.energy(x, y, z, *lists)[0], f0, rtol=1e-12, atol=1e-9)
     ctx.close()
+
+
+# Pairs exactly half an edge apart inside the cutoff: 64 equal waters on a 4 A
+# lattice along x (edge 16 A, cutoff 9 A), moved along y and z, so that the image
+# index is a tie for atoms of one kind two cells apart.
+def test_half_edge_images():
+    wb = configs.build(dict(configs.COMMON, name="lattice", n_waters=64, L=16.0, seed=3, grid=16,
+                            timeStep=0.002, precision="fp64", cutOff=9.0, cutOn=7.5, delr=0.5,
+                            alpha=0.35))
+    rng = np.random.default_rng(3)
+    cell = np.stack(np.meshgrid(*[np.arange(4)] * 3, indexing="ij"), -1).reshape(64, 3) * 4.0 - 6.0
+    cell[:, 1:] += rng.uniform(-0.4, 0.4, (64, 2))
+    mol = np.stack([wb.x[:3], wb.y[:3], wb.z[:3]], 1)
+    mol = np.round((mol - mol[0]) * 2**20) / 2**20      # differences along x are exact
+    p = (cell[:, None, :] + mol[None]).reshape(-1, 3)
+    x, y, z = (np.ascontiguousarray(p[:, k]) for k in range(3))
+    ties = np.abs(x[:, None] - x[None]) == 8.0
+    assert ties.sum() > 1000
+    o = O.OracleSystem(wb)
+    nl, np_, no = o.build_list(x, y, z)
+    ctx = M.Context(wb)
+    ctx.makelist(x.copy(), y.copy(), z.copy())
+    for elec in (2, 4):
+        f_o, _ = o.nonbond_energy(elec, x, y, z)
+        assert relerr(ctx.nonbond_energy(elec, x, y, z, nl, np_, no)[0], f_o) < 1e-12
+    f_o, e_o = o.energy(x, y, z)
+    assert relerr(ctx.energy(x, y, z, nl, np_, no)[0], f_o) < 1e-12
+    ctx.upload(x, y, z, *[np.zeros(wb.n)] * 3)
+    e_d = ctx.initial_energy()
+    assert e_d.nInCut == e_o["nInCut"]
+    assert relerr(np.stack(ctx.download()[6:9]), f_o) < 1e-12
+    ctx.close()
