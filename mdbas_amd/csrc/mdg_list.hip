@@ -771,8 +771,22 @@ __device__ __forceinline__ void test_candidates(const MdgParams &P, const MdgBox
 // candidates; a large one fills the chip with one wavefront a cluster and is bound
 // by the predicate's FP64 issue.  Four wavefronts against one: 648 atoms (about 100
 // clusters) 16 : 46 us, 3,000 59 : 148, 30,000 (3,900 clusters) 194 : 196.
+// The four keep their finds in LDS, kmax each (a row's room, so a wavefront that
+// finds more has overflowed the list), and a longer cutoff then leaves fewer blocks
+// on a CU: split up to three rounds of the blocks that LDS holds at once.  Step with
+// a list build each (mixed, us), four against one: 15 A cutoff 21,000 atoms (2.8
+// rounds) 545 : 594, 30,000 (4) 648 : 618; 18 A 12,000 (2.1) 589 : 693, 18,000 (3.2)
+// 771 : 762, 24,000 (4.2) 855 : 748.
 #define SPLIT_NCLU 4096           // clusters up to which four wavefronts share one
-#define SPLIT_CAP 160            // finds a sharing wavefront keeps (else one wave redoes the cluster)
+static size_t split_lds(int kmax)
+{
+    return 4 * (size_t)kmax * (sizeof(unsigned long long) + sizeof(int));
+}
+static bool split_search(int nclu, int kmax)
+{
+    const size_t lds = split_lds(kmax), perCu = 160 * 1024 / lds;
+    return nclu <= SPLIT_NCLU && lds <= 64 * 1024 && (size_t)nclu <= 3 * 256 * perCu;
+}
 
 template <int SPLIT>
 __global__ void __launch_bounds__(256)
@@ -848,26 +862,22 @@ k_cluster_pairs(MdgParams P, MdgBox B, int keyLink, int nx, int ny, int nz, int 
     const PairSink out = {tmpJ + (long)I * kmax, tmpMask + (long)I * kmax, kmax};
     int found;
     if (SPLIT > 1) {
-        __shared__ int sJ[SPLIT][SPLIT_CAP], sn[SPLIT];
-        __shared__ unsigned long long sM[SPLIT][SPLIT_CAP];
+        extern __shared__ unsigned long long sM[];   // SPLIT rows of masks, then of indices
+        __shared__ int sn[SPLIT];
+        int *sJ = (int *)(sM + SPLIT * kmax) + wv * kmax;
         const int mine = search(wv * nrow / SPLIT, (wv + 1) * nrow / SPLIT,
-                                PairSink{sJ[wv], sM[wv], SPLIT_CAP});
+                                PairSink{sJ, sM + wv * kmax, kmax});
         if (lane == 0) sn[wv] = mine;
         __syncthreads();
-        int base = 0, over = 0;
+        int base = 0;
         found = 0;
         for (int w = 0; w < SPLIT; w++) {
             if (w < wv) base += sn[w];
             found += sn[w];
-            over |= sn[w] > SPLIT_CAP;
         }
-        if (over) {
-            if (wv == 0) search(0, nrow, out);
-        } else {
-            for (int k = lane; k < mine && base + k < kmax; k += 64) {
-                out.J[base + k] = sJ[wv][k];
-                out.mask[base + k] = sM[wv][k];
-            }
+        for (int k = lane; k < mine && base + k < kmax; k += 64) {
+            out.J[base + k] = sJ[k];
+            out.mask[base + k] = sM[wv * kmax + k];
         }
         if (wv > 0) return;
     } else {
@@ -1127,9 +1137,10 @@ int mdg_build_cluster_list(mdg_ctx *ctx)
         CG.rx = (int)(rl / (ctx->B.pa / C.nfx)) + 1;
         CG.ry = (int)(rl / (ctx->B.pb / C.nfy)) + 1;
     }
-    const bool split = nclu <= SPLIT_NCLU;
+    const bool split = split_search(nclu, C.kmax);
     hipLaunchKernelGGL(split ? k_cluster_pairs<4> : k_cluster_pairs<1>,
-                       dim3(split ? nclu : nblk(nclu, 4)), dim3(256), 0, ctx->stream, ctx->P,
+                       dim3(split ? nclu : nblk(nclu, 4)), dim3(256),
+                       split ? split_lds(C.kmax) : 0, ctx->stream, ctx->P,
                        ctx->B, ctx->keyLink, ctx->nlc[0], ctx->nlc[1], ctx->nlc[2], nclu,
                        C.bb, C.bbh, C.pk, ctx->hasFrozen,
                        ctx->frozen, ctx->exOff, ctx->exLst, ctx->exSpan, C.kmax, C.tmpCnt, C.tmpJ,

@@ -210,3 +210,30 @@ def test_half_edge_images():
     assert e_d.nInCut == e_o["nInCut"]
     assert relerr(np.stack(ctx.download()[6:9]), f_o) < 1e-12
     ctx.close()
+
+
+def pairset(nl, np_, no, n):
+    a, c = np.repeat(no, np_[no]).astype(np.int64), nl.astype(np.int64)
+    return np.sort(np.minimum(a, c) * n + np.maximum(a, c))
+
+
+def device_pairs(ctx):
+    pi, pj = ctx.list_pairs()
+    return np.sort(pi.astype(np.int64) * ctx.n + pj)
+
+
+# Cluster search with four wavefronts a cluster at cutoffs where one of them finds
+# several hundred entries.
+@pytest.mark.parametrize("nw,cut", [(1000, 14.5), (1500, 17.0), (2500, 18.0), (3000, 20.0)])
+def test_long_cutoff_lists(nw, cut):
+    wb = water(nw, cut, 0.5)
+    print("atoms", wb.n, "cutoff", cut, flush=True)
+    o = O.OracleSystem(wb)
+    x, y, z = wb.x.copy(), wb.y.copy(), wb.z.copy()
+    want = pairset(*o.build_list(x, y, z), wb.n)
+    ctx = M.Context(wb)
+    ctx.upload(x, y, z, wb.vx, wb.vy, wb.vz)
+    ctx.initial_energy()
+    print(ctx.list_stats(), flush=True)
+    assert np.array_equal(device_pairs(ctx), want)
+    ctx.close()
