@@ -248,18 +248,18 @@ __global__ void __launch_bounds__(256) k_m3_vv1_a(ShakeArgs A, SideWork S)
         m_drift(A, M);
         m_setup_r(A, B, g, M);
     }
-    const bool first = tri_first<BATCH>(A, g);
-    int nr = 0, saved[SHK_R] = {-1, -1, -1, -1};
+    const unsigned long long share = tri_share<BATCH>(A, g);
+    TriRing ring;
     for (;;) {
         double l[3];
         const bool ok = live ? m_lambda_r(B, M, l) : true;
-        const bool all = tri_all<BATCH>(!ok, first);
+        const bool all = tri_all<BATCH>(!ok, share);
         // one system: the wavefront's molecules share a stopping sweep
         const bool cv = BATCH ? ok : all;
         if (cv) bits.cur |= 1ull << (it & 63);
-        if (all) {
-            if (live) m_save<true>(A, g, M, nr & (SHK_R - 1));
-            tri_saved(saved, nr++, it);
+        if (ring.keep<BATCH>(all)) {
+            if (live) m_save<true>(A, g, M, ring.slot());
+            ring.put(it);
         }
         settled = settled || (cv && prev);
         prev = cv;
@@ -271,7 +271,7 @@ __global__ void __launch_bounds__(256) k_m3_vv1_a(ShakeArgs A, SideWork S)
     }
     tri_flush(bits, it >> 6);
     if (live) {
-        for (int q = 0; q < SHK_R; q++) A.ring[(long)SHK_R * g + q] = saved[q];
+        for (int q = 0; q < SHK_R; q++) A.ring[(long)SHK_R * g + q] = ring.saved[q];
     }
     tri_publish<BATCH>(A, g, bits, it, settled);
 }
@@ -360,17 +360,17 @@ __global__ void __launch_bounds__(256) k_m3_vv2_a(ShakeArgs A, FinArgs F, int fu
         m_setup_v(A, M);
     }
     const double tolvel = A.P.tolShake * A.P.rTimeStep;
-    const bool first = tri_first<BATCH>(A, g);
-    int nr = 0, saved[SHK_R] = {-1, -1, -1, -1};
+    const unsigned long long share = tri_share<BATCH>(A, g);
+    TriRing ring;
     for (;;) {
         double l[3];
         const bool ok = live ? m_lambda_v(M, tolvel, l) : true;
-        const bool all = tri_all<BATCH>(!ok, first);
+        const bool all = tri_all<BATCH>(!ok, share);
         const bool cv = BATCH ? ok : all;
         if (cv) bits.cur |= 1ull << (it & 63);
-        if (all) {
-            if (live) m_save<false>(A, g, M, nr & (SHK_R - 1));
-            tri_saved(saved, nr++, it);
+        if (ring.keep<BATCH>(all)) {
+            if (live) m_save<false>(A, g, M, ring.slot());
+            ring.put(it);
         }
         settled = settled || (cv && prev);
         prev = cv;
@@ -382,7 +382,7 @@ __global__ void __launch_bounds__(256) k_m3_vv2_a(ShakeArgs A, FinArgs F, int fu
     }
     tri_flush(bits, it >> 6);
     if (live) {
-        for (int q = 0; q < SHK_R; q++) A.ring[(long)SHK_R * g + q] = saved[q];
+        for (int q = 0; q < SHK_R; q++) A.ring[(long)SHK_R * g + q] = ring.saved[q];
     }
     tri_publish<BATCH>(A, g, bits, it, settled);
     if (!BATCH && fuse) mdg_block_partials<2>(facc, F.part);

@@ -139,52 +139,85 @@ __device__ __forceinline__ void tri_flush(TriBits &b, int word)
     b.cur = 0;
 }
 
-// Whether this sweep can be the stopping sweep as far as this wavefront knows:
-// all its molecules are converged, in a batch all those of this lane's replica
-// (a wavefront holds at most the end of one replica and the start of the next;
-// first: whether the lane's is the first of the two).
+// The lanes whose molecules stop together with this lane's: the wavefront's, in a
+// batch those of its replica (idle lanes are their own share).  One pass per replica
+// in the wavefront, once a stage.
 template <bool BATCH>
-__device__ __forceinline__ bool tri_all(bool bad, bool first)
+__device__ inline unsigned long long tri_share(const ShakeArgs &A, int g)
 {
-    if (!BATCH) return __builtin_amdgcn_ballot_w64(bad) == 0;
-    const unsigned long long b0 = __builtin_amdgcn_ballot_w64(bad && first);
-    const unsigned long long b1 = __builtin_amdgcn_ballot_w64(bad && !first);
-    return (first ? b0 : b1) == 0;
+    if (!BATCH) return ~0ull;
+    const int r = g < A.nGrp ? A.grep[g] : -1;
+    unsigned long long share = 0, todo = __builtin_amdgcn_ballot_w64(true);
+    while (todo) {
+        const int lead = __builtin_amdgcn_readlane(r, __builtin_ctzll(todo));
+        const unsigned long long m = __builtin_amdgcn_ballot_w64(r == lead);
+        if (r == lead) share = m;
+        todo &= ~m;
+    }
+    return share;
 }
 
+// Whether this sweep can be the stopping sweep as far as this wavefront knows: every
+// molecule of the lane's share is converged.
 template <bool BATCH>
-__device__ __forceinline__ bool tri_first(const ShakeArgs &A, int g)
+__device__ __forceinline__ bool tri_all(bool bad, unsigned long long share)
 {
-    if (!BATCH) return true;
-    const int r = A.grep[min(g, A.nGrp - 1)];
-    return r == __builtin_amdgcn_readfirstlane(r);
+    const unsigned long long b = __builtin_amdgcn_ballot_w64(bad);
+    return BATCH ? (b & share) == 0 : b == 0;
 }
 
-// Notes that the nr-th wavefront-converged sweep was it (a ring of SHK_R: a
-// residual that passes through zero converges at a lone sweep, which can be the
-// global stop, before it settles).
-__device__ __forceinline__ void tri_saved(int (&saved)[SHK_R], int nr, int it)
-{
+// The sweeps whose states part A keeps for one share, in a ring of SHK_R slots: those
+// at which the share was converged (a residual that passes through zero converges at
+// a lone sweep, which can be the global stop, before it settles), up to the second of
+// two in a row.  A wavefront of one system ends there; one of a batch sweeps on for its
+// other replicas, and states from then on would push out the ones the stop needs (512
+// replicas of 40 to 52 molecules, a molecule per lane: 298 us a step, with them 340).
+struct TriRing {
+    int saved[SHK_R] = {-1, -1, -1, -1}, nr = 0;
+    bool prev = false, done = false;   // batch
+
+    // Whether this sweep's state is kept.
+    template <bool BATCH>
+    __host__ __device__ __forceinline__ bool keep(bool all)
+    {
+        if (!BATCH) return all;
+        const bool k = all && !done;
+        done = done || (all && prev);
+        prev = all;
+        return k;
+    }
+
+    // The slot of the next state, and that it was sweep it's.
+    __host__ __device__ __forceinline__ int slot() const { return nr & (SHK_R - 1); }
+    __host__ __device__ __forceinline__ void put(int it)
+    {
 #pragma unroll
-    for (int q = 0; q < SHK_R; q++)
-        if (q == (nr & (SHK_R - 1))) saved[q] = it;
-}
+        for (int q = 0; q < SHK_R; q++)
+            if (q == slot()) saved[q] = it;
+        nr++;
+    }
+};
 
-// The latest saved sweep of molecule g that is not past C, and its slot; -1
-// when there is none.
-__device__ inline int tri_resume(const ShakeArgs &A, int g, int C, int &slot)
+// The latest saved sweep of a ring that is not past C, and its slot; -1 when there
+// is none.
+__host__ __device__ inline int tri_resume(const int *ring, int C, int &slot)
 {
     int at = -1;
     slot = 0;
 #pragma unroll
     for (int q = 0; q < SHK_R; q++) {
-        const int s = A.ring[(long)SHK_R * g + q];
+        const int s = ring[q];
         if (s <= C && s > at) {
             at = s;
             slot = q;
         }
     }
     return at;
+}
+
+__device__ inline int tri_resume(const ShakeArgs &A, int g, int C, int &slot)
+{
+    return tri_resume(A.ring + (long)SHK_R * g, C, slot);
 }
 
 template <bool BATCH>

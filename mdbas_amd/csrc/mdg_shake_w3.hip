@@ -258,8 +258,9 @@ __global__ void __launch_bounds__(256) k_w3_vv1_a(ShakeArgs A, SideWork S)
     const double ddsq = q_ddsq(Q);
     TriBits bits;
     tri_bits_init(bits);
-    const bool first = tri_first<BATCH>(A, g);
-    int it = 0, nr = 0, saved[SHK_R] = {-1, -1, -1, -1};
+    const unsigned long long share = tri_share<BATCH>(A, g);
+    TriRing ring;
+    int it = 0;
     bool prev = false, settled = false;
     // until every molecule of the wavefront was converged at two consecutive
     // checks (the wavefront's time is its slowest molecule's)
@@ -271,9 +272,9 @@ __global__ void __launch_bounds__(256) k_w3_vv1_a(ShakeArgs A, SideWork S)
         const bool bad = Q.k < 3 && !(fabs(e) < Q.T.thr);
         const bool cv = q_conv<BATCH>(__builtin_amdgcn_ballot_w64(bad));
         if (cv) bits.cur |= 1ull << (it & 63);
-        if (tri_all<BATCH>(bad, first)) {
-            q_save<true>(A, g, Q, nr & (SHK_R - 1));
-            tri_saved(saved, nr++, it);
+        if (ring.keep<BATCH>(tri_all<BATCH>(bad, share))) {
+            q_save<true>(A, g, Q, ring.slot());
+            ring.put(it);
         }
         settled = settled || (cv && prev);
         prev = cv;
@@ -286,7 +287,7 @@ __global__ void __launch_bounds__(256) k_w3_vv1_a(ShakeArgs A, SideWork S)
     }
     tri_flush(bits, it >> 6);
     if (Q.k == 0) {
-        for (int q = 0; q < SHK_R; q++) A.ring[(long)SHK_R * g + q] = saved[q];
+        for (int q = 0; q < SHK_R; q++) A.ring[(long)SHK_R * g + q] = ring.saved[q];
     }
     tri_publish<BATCH>(A, g, bits, it, settled);
 }
@@ -389,8 +390,9 @@ __global__ void __launch_bounds__(256) k_w3_vv2_a(ShakeArgs A, FinArgs F, int fu
     const double tolvel = A.P.tolShake * A.P.rTimeStep;
     TriBits bits;
     tri_bits_init(bits);
-    const bool first = tri_first<BATCH>(A, g);
-    int it = 0, nr = 0, saved[SHK_R] = {-1, -1, -1, -1};
+    const unsigned long long share = tri_share<BATCH>(A, g);
+    TriRing ring;
+    int it = 0;
     bool prev = false, settled = false;
     // the check is the sweep's own max |lambda| (shake.c:421); every sweep
     // that is not the last one checked is applied, because the reference's
@@ -400,9 +402,9 @@ __global__ void __launch_bounds__(256) k_w3_vv2_a(ShakeArgs A, FinArgs F, int fu
         const bool bad = !(fabs(l) < tolvel);
         const bool cv = q_conv<BATCH>(__builtin_amdgcn_ballot_w64(bad));
         if (cv) bits.cur |= 1ull << (it & 63);
-        if (tri_all<BATCH>(bad, first)) {
-            q_save<false>(A, g, Q, nr & (SHK_R - 1));
-            tri_saved(saved, nr++, it);
+        if (ring.keep<BATCH>(tri_all<BATCH>(bad, share))) {
+            q_save<false>(A, g, Q, ring.slot());
+            ring.put(it);
         }
         settled = settled || (cv && prev);
         prev = cv;
@@ -414,7 +416,7 @@ __global__ void __launch_bounds__(256) k_w3_vv2_a(ShakeArgs A, FinArgs F, int fu
     }
     tri_flush(bits, it >> 6);
     if (Q.k == 0) {
-        for (int q = 0; q < SHK_R; q++) A.ring[(long)SHK_R * g + q] = saved[q];
+        for (int q = 0; q < SHK_R; q++) A.ring[(long)SHK_R * g + q] = ring.saved[q];
     }
     tri_publish<BATCH>(A, g, bits, it, settled);
     if (!BATCH && fuse) mdg_block_partials<2>(facc, F.part);

@@ -35,3 +35,33 @@ def test_reference_list_partials_fit(tmp_path):
         assert group >= 4
         assert group * blocks >= n > group * (blocks - 1)
         assert blocks * 6 <= region, (n, blocks)
+
+
+# Sweeps at which one replica's molecules of a wavefront are converged, while the
+# wavefront sweeps on to the end for another replica; for a stop at sweep C, the
+# latest state that part A kept.
+@pytest.mark.parametrize("conv,end,stops", [
+    (range(10, 41), 40, {9: -1, 10: 10, 11: 11, 12: 11, 25: 11, 40: 11}),
+    ([3, 5, *range(9, 60)], 59, {2: -1, 3: 3, 4: 3, 5: 5, 9: 9, 10: 10, 50: 10}),
+    ([10, 11, 12, *range(15, 30)], 29, {10: 10, 12: 11, 15: 11, 29: 11}),
+    ([0, 1], 1, {0: 0, 1: 1}),
+    ([1, 3, 5, 7, 9, 10], 10, {1: -1, 4: -1, 5: 5, 10: 10}),     # the ring holds four
+])
+def test_shake_states_for_a_replica(tmp_path, conv, end, stops):
+    conv = set(conv)
+    bits = ", ".join("1" if k in conv else "0" for k in range(end + 1))
+    body = f"const int conv[] = {{{bits}}};\n" """
+    TriRing r;
+    int at[SHK_R] = {-1, -1, -1, -1};
+    for (int k = 0; k < (int)(sizeof conv / sizeof *conv); k++) {
+        if (!r.keep<true>(conv[k])) continue;
+        at[r.slot()] = k;
+        r.put(k);
+    }
+    """ + f"for (int c : {{{', '.join(map(str, stops))}}}) " """{
+        int slot;
+        const int s = tri_resume(r.saved, c, slot);
+        printf("%d %d %d\\n", c, s, s < 0 ? -1 : at[slot]);
+    }"""
+    for c, s, kept in run_host(tmp_path, body, includes=("mdg_shake_tri.h",)):
+        assert s == kept == stops[c], (c, s, kept)

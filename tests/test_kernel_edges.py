@@ -237,3 +237,34 @@ def test_long_cutoff_lists(nw, cut):
     print(ctx.list_stats(), flush=True)
     assert np.array_equal(device_pairs(ctx), want)
     ctx.close()
+
+
+# Replicas small enough that a wavefront holds three and more of them, their SHAKE
+# sweeps unequal (66 to 600 K), against a single box each.
+@pytest.mark.parametrize("spread", [0, 1, 2])
+def test_small_replicas(spread):
+    boxes = []
+    for k, (nw, temp) in enumerate([(30, 66.0), (45, 600.0), (33, 100.0), (52, 300.0), (30, 450.0),
+                                    (38, 150.0), (64, 300.0), (31, 500.0)]):
+        boxes.append(configs.build(dict(
+            configs.COMMON, name=f"r{k}", n_waters=nw, L=(nw / 0.0334) ** (1 / 3), seed=50 + k,
+            grid=16, cutOff=4.3, cutOn=2.8, delr=0.3, alpha=0.35, temp=temp, timeStep=0.0005,
+            precision="fp64")))
+    print("spread", spread, [b.n for b in boxes], flush=True)
+    b = M.BatchContext(boxes, precision=M.MDG_FP64)
+    b.set_launch(**dict(b.get_launch(), shake_spread=spread))
+    b.upload_boxes()
+    b.initial_energy()
+    rb = M.batch_records(b.run(6), b.R)
+    sb = [b.split(a) for a in b.download()[:6]]
+    b.close()
+    for r, wb in enumerate(boxes):
+        c = M.Context(wb)
+        c.upload(wb.x, wb.y, wb.z, wb.vx, wb.vy, wb.vz)
+        c.initial_energy()
+        rs = M.records_to_dict(c.run(6))
+        ss = c.download()[:6]
+        c.close()
+        for k in ("tot", "kin", "virshake"):
+            assert np.allclose(rb[k][:, r], rs[k], rtol=1e-10, atol=1e-10 * abs(rs["pot"][0])), k
+        assert max(np.abs(sb[k][r] - ss[k]).max() for k in range(6)) < 1e-9
