@@ -268,3 +268,121 @@ def test_small_replicas(spread):
         for k in ("tot", "kin", "virshake"):
             assert np.allclose(rb[k][:, r], rs[k], rtol=1e-10, atol=1e-10 * abs(rs["pot"][0])), k
         assert max(np.abs(sb[k][r] - ss[k]).max() for k in range(6)) < 1e-9
+
+
+def lists_equal(got, want):
+    return all(np.array_equal(a, b) for a, b in zip(got, want))
+
+
+def frozen_steps(ctx, o, wb, x, y, z, nsteps=3):
+    """A few device-resident FP64 steps with frozen atoms (no force and no velocity
+    after the energies, utils.c:131-153) against the oracle's stages (1e-9 A over
+    the rounding of a few steps, as the batch tests)."""
+    s = [x.copy(), y.copy(), z.copy(), wb.vx.copy(), wb.vy.copy(), wb.vz.copy()]
+    ctx.upload(*s)
+    ctx.initial_energy()
+    ctx.run(nsteps)
+    g = ctx.download()
+
+    def forces():
+        f, _ = o.energy(*s[:3])
+        for a in (*s[3:], *f):
+            a[wb.frozen != 0] = 0.0
+        return f
+
+    f = forces()
+    for _ in range(nsteps):
+        assert o.vv(1, *s, f)[0] == 0
+        f = forces()
+        assert o.vv(2, *s, f)[0] == 0
+    assert relerr(np.stack(g[6:9]), f) < 1e-9
+    assert max(np.abs(a - b).max() for a, b in zip(g[:6], s)) < 1e-9
+
+
+# Every third molecule frozen, through both list builders (link cells from 136
+# molecules on), the device list, a batch, and a step; flags that only makelist is
+# given, and their going away.
+@pytest.mark.parametrize("nw", [43, 136])
+def test_frozen_atoms(nw):
+    wb = water(nw, 3.4, 0.4)
+    free = M.Context(wb)
+    x, y, z = wb.x.copy(), wb.y.copy(), wb.z.copy()
+    o_free = O.OracleSystem(wb)
+    want_free = [a.copy() for a in o_free.build_list(x, y, z)]
+    assert free.key_link == o_free.keyLink == (1 if nw == 136 else 0)
+    wb.frozen = np.repeat((np.arange(nw) % 3 == 0).astype(np.int32), 3)
+    wb.vx, wb.vy, wb.vz = (np.where(wb.frozen, 0.0, v) for v in (wb.vx, wb.vy, wb.vz))
+    o = O.OracleSystem(wb)
+    want = [a.copy() for a in o.build_list(x, y, z)]
+    assert len(want[0]) < len(want_free[0])
+    # the flags come with makelist alone, then without them
+    pos = lambda: (x.copy(), y.copy(), z.copy())  # noqa: E731
+    assert lists_equal(free.makelist(*pos())[:3], want)
+    wb.frozen, flags = np.zeros_like(wb.frozen), wb.frozen
+    free.ctrl.newjob = 1
+    assert lists_equal(free.makelist(*pos())[:3], want_free)
+    free.close()
+    wb.frozen = flags
+    ctx = M.Context(wb)
+    assert lists_equal(ctx.makelist(*pos())[:3], want)
+    frozen_steps(ctx, o, wb, x, y, z)
+    ctx.upload(x, y, z, wb.vx, wb.vy, wb.vz)
+    ctx.initial_energy()
+    assert np.array_equal(device_pairs(ctx), pairset(*want, wb.n))
+    ctx.close()
+    if nw == 43:
+        b = M.BatchContext([wb, wb])
+        b.upload_boxes()
+        b.initial_energy()
+        one = pairset(*want, 2 * wb.n)
+        assert np.array_equal(device_pairs(b),
+                              np.sort(np.concatenate([one, one + wb.n * (2 * wb.n + 1)])))
+        b.close()
+
+
+# Triclinic boxes (the drop-in calls take them): both list builders, the pair loop,
+# meshes of the in-LDS convolution and of the library's transforms, and SHAKE.
+@pytest.mark.parametrize("nw,grid", [(60, 24), (60, 22), (136, 24)])
+def test_triclinic_boxes(nw, grid, monkeypatch):
+    wb = water(nw, 3.4, 0.4, grid=grid)
+    L = wb.L
+    cell = np.array([[L, 0, 0], [0.12 * L, L, 0], [-0.09 * L, 0.07 * L, L]])
+    p = np.stack([wb.x, wb.y, wb.z], 1).reshape(-1, 3, 3)
+    rel = p - p[:, :1]
+    rel -= L * np.round(rel / L)
+    p = ((p[:, :1] / L) @ cell + rel).reshape(-1, 3)
+    x, y, z = (np.ascontiguousarray(p[:, k]) for k in range(3))
+    monkeypatch.setattr(O, "make_box", lambda edge: O.box_from9(cell.ravel(), 3))
+    made = M.reference_structs
+
+    def structs(*a):
+        s = made(*a)
+        s[2].type = 3
+        (s[2].a1, s[2].a2, s[2].a3, s[2].b1, s[2].b2, s[2].b3, s[2].c1, s[2].c2,
+         s[2].c3) = cell.ravel()
+        return s
+
+    monkeypatch.setattr(M, "reference_structs", structs)
+    print("triclinic", wb.n, "atoms, mesh", grid, flush=True)
+    o = O.OracleSystem(wb)
+    ctx = M.Context(wb)
+    assert ctx.key_link == o.keyLink == (1 if nw == 136 else 0)
+    g = [x.copy(), y.copy(), z.copy()]
+    want = [a.copy() for a in o.build_list(x, y, z)]
+    assert lists_equal(ctx.makelist(*g)[:3], want)
+    assert lists_equal(g, (x, y, z))
+    for elec in (2, 4):
+        f_o, _ = o.nonbond_energy(elec, x, y, z)
+        assert relerr(ctx.nonbond_energy(elec, x, y, z, *want)[0], f_o) < 1e-12
+    er, fr, st, vr = o.spme(x, y, z)
+    eg, fg, sg, vg = ctx.spme_energy(x, y, z)
+    assert eg == pytest.approx(er, rel=1e-12) and relerr(fg, fr) < 1e-11
+    f_o, _ = o.energy(x, y, z)
+    assert relerr(ctx.energy(x, y, z, *want)[0], f_o) < 1e-12
+    s_o = [x, y, z, wb.vx.copy(), wb.vy.copy(), wb.vz.copy()]
+    s_g = [a.copy() for a in s_o]
+    for stage in (1, 2):
+        assert o.vv(stage, *s_o, f_o)[0] == 0
+        ctx.vv_integrate(stage, *s_g, f_o.copy())
+        assert max(np.abs(a - b).max() for a, b in zip(s_o, s_g)) < 1e-12
+    ctx.close()
