@@ -19,6 +19,18 @@ __device__ __forceinline__ double mdg_rcp64(double x)
     return __builtin_fma(y, __builtin_fma(h, h, h), y);
 }
 
+// a / b for normal b and quotients, from a reciprocal and one correction by the
+// remainder a - q b, which is exact.  The reciprocal's error (0.5 ulp and 2^-24 of
+// one) times the remainder (at most an ulp or two of q) is below 2^-51 ulp of q, so
+// the result is the correctly rounded quotient unless the exact one lies that close
+// to a midpoint of two doubles; then it is one of the two.
+__device__ __forceinline__ double mdg_div64(double a, double b)
+{
+    const double y = mdg_rcp64(b);
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+
 // 1/sqrt(x) for normal x > 0, by the same third-order step
 // y (1 + h/2 + 3 h^2 / 8), h = 1 - x y^2; r receives sqrt(x), x y with one
 // correction for its rounding.

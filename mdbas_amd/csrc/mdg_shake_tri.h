@@ -8,17 +8,18 @@
 // the corrections).  Atom k belongs to constraints k and k - 1 and moves along
 // their vectors dd of the stage's start.
 //
-// The iterates follow the reference's loops (shake.c:262-332, 378-436) bit for
-// bit: they feed the rounding of each moved position or velocity back into the
+// The iterates follow the reference's loops (shake.c:262-332, 378-436) rounding by
+// rounding: they feed the rounding of each moved position or velocity back into the
 // next multiplier, so anything less differs by that rounding (over dt, in the
-// velocities: 3e-11 A/ps at dt = 1 fs).  What a sweep leaves out is exact:
+// velocities: 3e-11 A/ps at dt = 1 fs).  What a sweep leaves out is exact, the
+// division up to quotients next to a rounding midpoint:
 //  * the factor 1/2 of the position multiplier and the 1/nAtConst sit in the
 //    atoms' factors (powers of two for the two constraints of an atom);
 //  * an atom's own multiplier needs no move between lanes, and of the other
 //    constraint only the multiplier moves;
 //  * divisions are a reciprocal (of a constant, in stage 2) and one correction
-//    by the remainder, which is exact, so the quotient is the correctly
-//    rounded one (the reciprocal is within an ulp).
+//    by the remainder, which is exact: mdg_div64, and how far that is the
+//    correctly rounded quotient.
 // About 65 instructions a position sweep and 40 a velocity sweep where there
 // were 110 and 80.
 //
@@ -27,15 +28,6 @@
 #pragma once
 #include "mdg_shake.h"
 #include "mdg_math64.h"
-
-// a / b from a reciprocal y of b within an ulp: the remainder a - q b is exact,
-// so the corrected quotient is the correctly rounded one.
-__device__ __forceinline__ double tri_div(double a, double b)
-{
-    const double y = mdg_rcp64(b);
-    const double q = a * y;
-    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
-}
 
 // The constant vector utils.c:38-80 subtracts from a bond vector: a bond (about
 // an angstrom) keeps its image over the sweeps of a stage, and d - shift is
@@ -76,7 +68,7 @@ __device__ __forceinline__ double tri_lambda(const MdgBox &B, const TriR &T, dou
         r2 = dx * dx + dy * dy + dz * dz;
     }
     e = r2 - T.rc2;
-    return tri_div(e, T.K * (ddx * dx + ddy * dy + ddz * dz));
+    return mdg_div64(e, T.K * (ddx * dx + ddy * dy + ddz * dz));
 }
 
 // Atom k's position and velocity.
