@@ -8,8 +8,9 @@ passed without being checked.  Its stop sweep is then the first sweep at
 which every group passed or had stopped, and the second kernel raises
 MDG_ESHAKE_ORDER when some group that had stopped fails the test at that
 sweep.  For one system of three-site molecules the stop is per wavefront of
-16 molecules (all of them at two consecutive passing sweeps at once); in a
-replica batch it is per molecule.
+16 molecules (all of them at two consecutive passing sweeps at once).  In a
+replica batch a wavefront goes on until each of its molecules has passed at
+two consecutive sweeps, checking them all until then.
 
 Each constraint group's iterates depend on that group alone, so the
 oracle's global sweeps give every group's pass/fail history up to C.  The
@@ -73,6 +74,20 @@ def device_stop(cg, width=1):
     return stop, not cg[stop].all()
 
 
+def batch_stop(cg, width):
+    """The rule of a replica batch, for one replica: `width` groups of a
+    wavefront are checked until the last of them has passed twice in a row;
+    sweeps after that count as passed."""
+    bits = cg.copy()
+    for lo in range(0, cg.shape[1], width):
+        both = cg[1:, lo:lo + width] & cg[:-1, lo:lo + width]
+        if both.any(0).all():
+            end = int(both.argmax(0).max()) + 1
+            bits[end + 1:, lo:lo + width] = True
+    stop = int(np.flatnonzero(bits.all(1))[0])
+    return stop, not cg[stop].all()
+
+
 def trajectory_histories(cfg, nsteps):
     wb = configs.build(cfg)
     o = O.OracleSystem(wb)
@@ -127,6 +142,13 @@ def test_device_rule_finds_the_reference_stop(histories, width):
     assert redivergent == 0
 
 
+def test_batch_rule_finds_the_reference_stop(histories):
+    name, hs = histories
+    for step, stage, cg in hs:
+        for width in (1, WAVE, 64):
+            assert batch_stop(cg, width) == (cg.shape[0] - 1, False), (name, step, stage, width)
+
+
 def test_replay_raises_on_a_redivergent_group():
     """Group 0 passes at sweeps 1 and 2, fails at 3 and 4, passes from 5;
     group 1 passes from sweep 3.  The device stops group 0 after sweep 2 and
@@ -139,6 +161,9 @@ def test_replay_raises_on_a_redivergent_group():
     # before sweep 5, so the checked bits stand and sweep 5 is taken, as
     # the reference takes it
     assert device_stop(cg, 2) == (5, False)
+    # in a batch's wavefront group 0 is checked until group 1 settles at
+    # sweep 4, which finds its failures
+    assert batch_stop(cg, 2) == (5, False)
 
 
 def test_replay_keeps_a_late_group():
