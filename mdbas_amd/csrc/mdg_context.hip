@@ -965,6 +965,7 @@ static int upload_ref_list(mdg_ctx *ctx, MdgXfer &X, std::vector<long> &off, con
     R.count = total;
     X.put(R.off, off.data(), n + 1);
     X.put(R.neighOrder, neighOrder, n);
+    RETCHK(X.check(ctx));   // before a copy from the caller's list is under way
     return h2d(ctx, R.neighList, neighList, total);
 }
 

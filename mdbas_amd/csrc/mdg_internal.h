@@ -221,6 +221,7 @@ struct MdgXfer {
     }
     // a device array to clear, on the way up
     template <typename T> void zero(T *dev, size_t cnt) { add(dev, nullptr, cnt * sizeof(T)); }
+    int check(struct mdg_ctx *ctx) const;   // the arrays are all there
     int up(struct mdg_ctx *ctx);
     int fetch(struct mdg_ctx *ctx, int nfirst);
     int deliver(struct mdg_ctx *ctx);

@@ -49,8 +49,7 @@ void MdgXfer::add(void *dev, void *host, size_t bytes)
     if (host || !in) total += (bytes + 15) & ~(size_t)15;
 }
 
-// Whether the segments go through the pinned buffer (else directly).
-int MdgXfer::prepare(mdg_ctx *ctx)
+int MdgXfer::check(mdg_ctx *ctx) const
 {
     if (full) {
         ctx->err = "too many arrays in one transfer";
@@ -60,6 +59,13 @@ int MdgXfer::prepare(mdg_ctx *ctx)
         ctx->err = "a host array of the call is missing";
         return MDG_EARG;
     }
+    return MDG_OK;
+}
+
+// Whether the segments go through the pinned buffer (else directly).
+int MdgXfer::prepare(mdg_ctx *ctx)
+{
+    RETCHK(check(ctx));
     packed = total <= XFER_MAX;
     for (int k = 0; k < n; k++)
         if (((uintptr_t)seg[k].dev & 15) || (seg[k].bytes & 3) || seg[k].bytes > XFER_MAX)
