@@ -291,7 +291,7 @@ struct mdg_ctx {
     int *ctrl = nullptr;         // device control words (see CTRL_*)
     double *shkScr = nullptr, *shkVir = nullptr;   // SHAKE state window (mdg_integrate.hip)
     int *shkFirst = nullptr, *shkKend = nullptr;
-    int *shkRing = nullptr;      // per group: the sweeps in the two ring slots
+    int *shkRing = nullptr;      // three-site groups: the sweeps in the SHK_R ring slots
     unsigned long long *shkMask = nullptr;   // [stage 1 | stage 2][SHK_MASKW]
     bool shakeW3 = false;        // all groups are three-site molecules
     // exclusions (CSR; symmetric for link cells, ordered otherwise)
@@ -635,10 +635,13 @@ void mdg_params_from(const MDG_CTRL *ctrl, const MDG_PARAM *p, MdgParams &P);
 // records: per-block partials [eElec, eVdw, virElec, virVdw, nIn, nListed]
 // into part, mdg_ref64_blocks(n) rows.  A block takes mdg_ref64_group(n) rows
 // of the list: whole rounds of the 256 CUs (a block fills one) with at most 32
-// rows a block, beyond which a group's distinct j outgrow its LDS table, and at
-// least 4, below which rows would share too few j to collect.  Above 1.4 million
-// atoms the groups grow instead of their number: the partials have one region
-// of epart.
+// rows a block, and at least 4, below which rows would share too few j to collect.
+// More rows share more of their j (at 30,000 atoms and 12 A, 32 rows touch about
+// 1,040 of them and 118 rows 1,560, of 4,096 places), and the cap of 32 costs large
+// systems time: us a call at caps of 32, 64, 128 and 480 rows, 9 A cutoff, 9,000
+// atoms 66, 52, 52, 228, 90,000 atoms 328, 264, 243, 266; 12 A, 3,000 atoms 58, 58,
+// 58, 572, 30,000 atoms 249, 218, 173, 479.  Above 1.4 million atoms the groups grow
+// instead of their number: the partials have one region of epart.
 inline int mdg_ref64_group(int n)
 {
     const int rounds = nblk(n, 256 * 32);

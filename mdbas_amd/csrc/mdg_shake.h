@@ -4,13 +4,13 @@
 #include "mdg_internal.h"
 #include "mdg_side.h"
 
-// Window of SHAKE states kept per group around its first convergence, and
-// a ring of SHK_R for the last sweeps at which a whole wavefront was
-// converged.
+// SHAKE states kept between a stage's two kernels.  Generic groups: slot 0 the
+// start, 1 to SHK_W a window after the first convergence, SHK_W + 1 the end.
+// Three-site molecules: a ring of the last SHK_R sweeps at which the molecules that
+// stop together were converged (TriRing), in slots 0 to SHK_R - 1.
 #define SHK_W 8
 #define SHK_R 4
-// [0] start, [1..W] window, [W+1] end, [W+2 .. W+1+R] ring
-#define SHK_SLOTS (SHK_W + 2 + SHK_R)
+#define SHK_SLOTS (SHK_W + 2)     // >= SHK_R
 #define SHK_MASKW 4               // 256 sweep indices
 
 struct ShakeArgs {
@@ -35,7 +35,7 @@ struct ShakeArgs {
     double *virScr;       // SHAKE virial at those states: [SHK_SLOTS][nGrp] for generic
                           // groups, [SHK_SLOTS][nGrp][3] (per constraint) for three-site
     int *first, *kend;    // per group: first converged sweep, last checked sweep
-    int *ring;            // three-site kernels, per group: the sweep in each ring
+    int *ring;            // three-site kernels, per group: the sweep of each ring
                           // slot (SHK_R ints, -1 when empty)
     unsigned long long *mask;   // device-wide AND of converged-sweep bits
     // replica batch: box and mask per replica, replica per group, and the
