@@ -529,7 +529,7 @@ __device__ __forceinline__ double fp64_dist(const MdgBox &b, double &dx, double 
 // has few chunks of 32 entries, so its chunks are shorter (chunk_len).  Before,
 // with 32 entries a chunk, library sqrt / divide / erfc / exp and per-component
 // DPP sums: 648 atoms 47.7 us, now 8.4; 3,000 atoms 59 -> 43; 12,000 atoms
-// 185 -> 148.  The j atomics are a fifth of what is left.
+// 185 -> 137.  The j atomics are a fifth of what is left.
 template <bool BATCH, int ELEC>
 __global__ void __launch_bounds__(256) k_pair_fp64(ClusterArgs A)
 {
@@ -1441,7 +1441,7 @@ int mdg_prune_list(mdg_ctx *ctx)
 //   dE/dsig_i += 4 eps_i eps_j (12 s^11 - 6 s^5) S(r) / r (both atoms)
 // with s = (sig_i + sig_j) / r and S the switch of vdw.c:144-184 (1 below
 // cutOn).  Same wavefront layout, loads ahead and functions as k_pair_fp64; slot
-// sums go to fdx (q), fdy (eps), fdz (sig).  FP64 issue; 12,000 atoms 119 us (161
+// sums go to fdx (q), fdy (eps), fdz (sig).  FP64 issue; 12,000 atoms 122 us (161
 // with library functions, per-component sums and no loads ahead), 3,000 37.
 __global__ void __launch_bounds__(256) k_adj_cluster(ClusterArgs A)
 {
