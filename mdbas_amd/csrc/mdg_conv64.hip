@@ -284,7 +284,11 @@ k_conv_inv(ConvPlan C, const double2 *__restrict__ tw, const double2 *__restrict
     __syncthreads();
     conv_fft(C.y, a, b, t2, 1, mh, C.mMh, 1, mh);
     // Z[k] = X[k] + conj X[nz-k] + i exp(2 pi i k / m3) (X[k] - conj X[nz-k]);
-    // a real mesh's X[0] and X[nz] are real
+    // X[0] and X[nz] of a real mesh are real.  In a triclinic box the influence
+    // function differs between a point with an index m/2 and its negative, and their
+    // imaginary parts do not cancel: they belong to the imaginary part of the mesh,
+    // which the reference's complex transform carries and never reads
+    // (spme.c:593-646), so they are left out
     for (unsigned i = threadIdx.x; i < (unsigned)(m2 * nz); i += blockDim.x) {
         const unsigned j = conv_div(i, nz, C.mNz), k = i - j * nz;
         const double2 u = a[j * mh + k], w = a[j * mh + nz - k];

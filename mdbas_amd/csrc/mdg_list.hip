@@ -988,6 +988,12 @@ static int chunk_len(const mdg_ctx *ctx, int entries)
 //   FP64  9,000 atoms 207 (2,048) : 215, 24,000 351 (2,048) : 375;
 //   mixed 18,000 179 (2,048) : 173, 30,000 199 : 193, 90,000 391 (4,096) : 400,
 //   192,000 744 (4,096) : 770; 256 replicas 881 (16,384) : 956.
+// Batches of R replicas of 216 to 336 molecules (9 A), R = 8, 24, 64 and 200.  More
+// blocks against 1,024, pair first: FP64 (2,048) 273 : 274, 354 : 380, 582 : 614,
+// 1,448 : 1,592; mixed (16,384) 219 : 220, 251 : 249, 315 : 315, 523 : 559.  SPME
+// first against pair first, at those blocks: FP64 254 : 273, 339 : 354, 611 : 582,
+// 1,570 : 1,448; mixed 213 : 219, 240 : 251, 299 : 315, 508 : 523.  Batches keep pair
+// first, which is the better one for the large FP64 ones only; the tuner picks.
 static void default_launch(mdg_ctx *ctx)
 {
     if (ctx->tune.set) return;
